@@ -87,20 +87,21 @@ typedef struct sddc_plan sddc_plan;
 
 /* Launch-shape choices of a plan (no counterpart in the reference; the
  * autotuner varies them).  0 leaves a field to the library's default.
- *   chain_segment    rows per segment of the parity chains of the solves
- *                    (>= rows per chain: one segment, no join)
- *   solve_instances  instances per solve workgroup: 1, 2 or 4 (quad-lane
- *                    kernels), 3 (quad-lane, 2 per A4 workgroup and 4 per
- *                    NAB2 workgroup), 5 (as 3, the A4 chains with two
- *                    exchanges per row and one streamed block), 6 (as 5,
- *                    3 per A4 workgroup), 7 and 8 (as 5 with four and six
- *                    rows of operator data in flight), 9 (one instance per
- *                    A4 workgroup, two exchanges, six rows in flight), 10
- *                    (one instance per A4 workgroup, one exchange, four
- *                    rows in flight), 16 (MFMA kernel).  1-4 and 10 give the
- *                    same bits, as do 5-9; these two groups and 16 sum in
- *                    different orders (equal to rounding), so the choice is
- *                    fixed per plan
+ *   chain_segment    the form of the solves: at least the rows of a parity
+ *                    chain (N_fm/2), one sequential chain; fewer, the
+ *                    eigenbasis of the theta operator, in which every mode
+ *                    solves by itself (for small and medium batches; equal
+ *                    to rounding, about 2e-14 relative at N_fm = 512; an
+ *                    operator set whose blocks are no polynomials in that
+ *                    operator keeps the chains).  The value below N_fm/2
+ *                    has no further meaning
+ *   solve_instances  launch shape of the chains: 1, 2, 4, 5 four instances
+ *                    per workgroup; 6, 10 the same with six instead of four
+ *                    rows of operator data in flight; 3, 7 four per A4
+ *                    and eight per NAB2 workgroup; 9 as 3 with six rows in
+ *                    flight; 8 eight per workgroup; 16 eight per A4 and
+ *                    sixteen per NAB2 workgroup.  The same bits whatever
+ *                    the value
  *   sub_batches      graphs only: the batch is split into this many parts
  *                    (1-8), stepped on forked streams inside the graph (see
  *                    sddc_graph_create_multi), so that the latency-bound
@@ -187,14 +188,14 @@ int sddc_step(sddc_plan* plan, int B, const double* Ra, const double* Ra_s,
 /* sddc_step for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  No
  * counterpart in the reference.  The step's intermediates (suffix sums,
- * linear part, slabs, products, right-hand side, solve exit states) live in
+ * linear part, slabs, products, right-hand side) live in
  * one static device array of SDDC_STATIC_SCRATCH_BYTES per GPU, held from
  * the first plan created on that GPU until the process ends, not in the
  * plan's workspace; the call makes no hipMalloc, hipFree or other allocating
  * call, and B is not limited by the plan's reserved batch.  A batch whose
  * intermediates do not fit the array is refused with SDDC_ERR_INVALID (the
  * message gives how many instances of the class fit: 25 at N_r = 40,
- * N_fm = 512 in mixed precision, 23 in float64, with unsegmented chains).
+ * N_fm = 512 in mixed precision, 23 in float64).
  * Every call on one GPU uses
  * the same array: calls that overlap in time on one GPU (other streams,
  * other threads, other plans) race.  Results are the same bits as

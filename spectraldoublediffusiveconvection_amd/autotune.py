@@ -1,8 +1,8 @@
 """Autotuner of the plans' launch shapes.
 
 For one size class and batch size it times HIP-graph-replayed steps under each
-candidate launch shape (rows per chain segment of the solves, instances per
-solve workgroup, sub-batches on forked streams) and keeps the fastest.  The
+candidate launch shape (form of the solves, launch shape of their chains,
+sub-batches on forked streams) and keeps the fastest.  The
 graphs hold GRAPH_STEPS steps, as the benchmark's and the sweep's do: the
 sub-batch streams start together at every graph launch, so the length of the
 graph changes how much they overlap.  Results are stored in a JSON table
@@ -39,22 +39,37 @@ def bucket(B):
 
 
 def candidates(N_fm, B=1):
-    """Launch shapes tried for a class with N_fm modes (N_fm/2 rows per chain)
-    at batch B: quad-lane solves with 1, 2 or 4 instances per workgroup, the
-    mixed widths 3, 5 and 6 (2 per A4, 4 per NAB2 workgroup; 5 with the
-    two-exchange A4 chains, 6 with three of them per workgroup) and 9, 10
-    (one instance per A4 workgroup with deeper prefetch), from B = 16 on the
-    16-instance MFMA solve, and from B = 64 on batches split in 2 or 4 parts
-    on forked streams of the graph."""
+    """Launch shapes of a class with N_fm modes (N_fm/2 rows per chain) at
+    batch B: chain_segment n asks for the chains, a smaller one for the theta
+    eigenbasis; solve_instances 1, 2, 4, 5 stand for one launch shape of the
+    chains, as do 3, 7 and 6, 10 (sddc.h); from B = 16 on also 16, and from
+    B = 64 on batches split in 2 or 4 parts on forked streams of the graph.
+    tune_class times one of each launch (distinct)."""
     n = N_fm // 2
     segs = {n, max(8, 4 * math.ceil(2 * math.sqrt(n) / 4))}
-    if B < 64:   # short segments only pay off while the device is not full
+    if B < 64:
         segs.add(max(8, 4 * math.ceil(math.sqrt(n) / 4)))
     segs = sorted(segs)
     nbs = (1, 2, 3, 4, 5, 6, 9, 10, 16) if B >= 16 else (1, 2, 3, 4, 5, 6, 9, 10)
     subs = (1, 2, 4) if B >= 64 else (1,)
     return [{"chain_segment": m, "solve_instances": nb, "sub_batches": sb}
             for m in segs for nb in nbs for sb in subs]
+
+
+SAME_CHAIN_LAUNCH = {2: 1, 4: 1, 5: 1, 7: 3, 10: 6}
+
+
+def distinct(shapes, N_fm):
+    """The shapes without those that launch the same kernels as an earlier one."""
+    seen, out = set(), []
+    for t in shapes:
+        chains = t["chain_segment"] >= N_fm // 2
+        nb = t["solve_instances"]
+        key = (SAME_CHAIN_LAUNCH.get(nb, nb) if chains else 0, t["sub_batches"])
+        if key not in seen:
+            seen.add(key)
+            out.append(t)
+    return out
 
 
 def shape_key(t):
@@ -78,7 +93,7 @@ def spectral_per_group(N_fm, B, spectral_instances):
 def refine_class(table, N_fm, N_r, B, widths=(), precision="mixed", steps=GRAPH_STEPS,
                  margin=0.05, spectral=(), rounds=3):
     """Time the table's shape for one class and batch again beside variants
-    of it -- the given solve widths at the candidate segment lengths, and the
+    of it -- the given solve widths with each form of the solves, and the
     given spectral-stage instances per workgroup -- and keep the fastest; a
     new shape must win by `margin`.  The shapes are timed in `rounds`
     interleaved rounds and each keeps its best.  Repeated plans of one shape
@@ -180,7 +195,7 @@ def tune_class(N_fm, N_r, B, precision="mixed", steps=GRAPH_STEPS):
     """Best launch shape for one class and batch size: (tuning, {shape: µs})."""
     timings = {}
     best, best_t = None, float("inf")
-    for t in candidates(N_fm, B):
+    for t in distinct(candidates(N_fm, B), N_fm):
         us = time_shape(N_fm, N_r, B, precision, t, steps=steps)
         timings[shape_key(t)] = round(us, 2)
         if us < best_t:

@@ -19,7 +19,7 @@ CSRC = os.path.join(PKG, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libsddc.so")
-SOURCES = ["sddc_api.hip", "sddc_transform.hip", "sddc_spectral.hip", "sddc_solve.hip",
+SOURCES = ["sddc_api.hip", "sddc_transform.hip", "sddc_spectral.hip", "sddc_solve.hip", "sddc_theta_solve.hip",
            "sddc_krylov.hip", "sddc_newton_batch.hip"]
 ARCH = os.environ.get("SDDC_OFFLOAD_ARCH", "gfx950")
 

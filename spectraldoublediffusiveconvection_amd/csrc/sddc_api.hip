@@ -126,7 +126,7 @@ void free_tables(TableSet& t) {
 
 int launch_solve_ex(const Plan& p, int B, const double* G, long long gstride,
                     const long long goff[3], double* X, long long xstride,
-                    const long long xoff[3], double* Pout, int fields_mask, hipStream_t s);
+                    const long long xoff[3], double* Pout, int fields_mask, bool step, hipStream_t s);
 int launch_rhs_scaled(const Plan& p, int B, const void* F, const double* L, double scale,
                       double* G, hipStream_t s);
 
@@ -151,14 +151,12 @@ static int upload(T** dst, const T* src, size_t n) {
 }
 
 static void free_ws(Plan& p) {
-  void* bufs[] = {p.P, p.L, p.G, p.Xa, p.Xb, p.Pa, p.slabs, p.slabs2, p.F, p.rowval, p.params,
-                  p.solve_scratch, p.chain_EX};
+  void* bufs[] = {p.P, p.L, p.G, p.Xa, p.Xb, p.Pa, p.slabs, p.slabs2, p.F, p.rowval, p.params};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   p.P = p.L = p.G = p.Xa = p.Xb = p.Pa = nullptr;
   p.slabs = p.slabs2 = p.F = nullptr;
-  p.rowval = p.params = p.solve_scratch = p.chain_EX = nullptr;
-  p.ex_batch = 0;
+  p.rowval = p.params = nullptr;
   p.ws_bytes = 0;
   p.max_batch = 0;
 }
@@ -187,12 +185,6 @@ static int alloc_ws(Plan& p, int B) {
   if ((rc = A(&p.F, (size_t)B * 4 * N * rs))) return rc;
   if ((rc = A((void**)&p.rowval, (size_t)B * p.nr * 8))) return rc;
   if ((rc = A((void**)&p.params, (size_t)2 * B * 8))) return rc;
-  // sink of padded instances and rows: X at [0, N), P at [N, 2N), lanes from 2N
-  if ((rc = A((void**)&p.solve_scratch, (4 * N + 256) * 8))) return rc;
-  // segment exit states of the solve, for B rounded up to whole workgroups
-  const int exb = ((B + 3) / 4) * 4;
-  if ((rc = A((void**)&p.chain_EX, (size_t)exb * 6 * p.nseg * 2 * p.NRP * 8))) return rc;
-  p.ex_batch = exb;
   p.ws_bytes = total;
   p.max_batch = B;
   return SDDC_OK;
@@ -328,6 +320,7 @@ int sddc_plan_create_tuned(const sddc_operators* ops, int precision, int symmetr
   if ((rc = build_chain(p, ops, max_batch > 0 ? max_batch : 1,
                         tuning ? tuning->chain_segment : 0)))
     return bail(rc);
+  if (p.nseg > 1 && (rc = build_theta(p, ops))) return bail(rc);
   if ((rc = build_tables(p.tabM, p.M))) return bail(rc);
   if ((rc = build_tables(p.tabKE, 3 * p.K))) return bail(rc);
   if ((rc = alloc_ws(p, max_batch > 0 ? max_batch : 1))) return bail(rc);
@@ -502,7 +495,8 @@ int sddc_bsub(sddc_plan* plan, int B, int field, const double* g, double* f, voi
   if (field < 0 || field > 2) return fail(SDDC_ERR_INVALID, "field must be 0 (psi), 1 (T) or 2 (S)");
   const long long N = (long long)p.K * p.nr;
   const long long off[3] = {0, 0, 0};
-  return launch_solve_ex(p, B, g, N, off, f, N, off, nullptr, 1 << field, (hipStream_t)stream);
+  return launch_solve_ex(p, B, g, N, off, f, N, off, nullptr, 1 << field, false,
+                         (hipStream_t)stream);
 }
 
 static int step_once(Plan& p, int B, const double* Ra, const double* Ras, const double* src,
@@ -554,8 +548,6 @@ static Plan sub_plan(const Plan& p, int b0, int nb) {
   v.slabs2 = static_cast<char*>(p.slabs2) + b0 * 7 * N * sizeof(double);
   v.F = static_cast<char*>(p.F) + b0 * 4 * N * rs;
   v.rowval = p.rowval + (size_t)b0 * p.nr;
-  v.chain_EX = p.chain_EX + (size_t)b0 * 6 * p.nseg * 2 * p.NRP;
-  v.ex_batch = p.ex_batch - b0;
   v.max_batch = nb;
   return v;
 }
@@ -610,10 +602,6 @@ static Plan static_view(const Plan& p, int B, unsigned char* base, size_t* need)
   v.Xa = p.symmetric ? reinterpret_cast<double*>(take((size_t)B * 3 * N * 8)) : nullptr;
   v.slabs = take((size_t)B * 7 * N * 8);   // sized as the plan's workspace sizes it
   v.F = take((size_t)B * 4 * N * rs);
-  v.solve_scratch = reinterpret_cast<double*>(take((4 * N + 256) * 8));
-  const int exb = ((B + 3) / 4) * 4;
-  v.chain_EX = reinterpret_cast<double*>(take((size_t)exb * 6 * p.nseg * 2 * p.NRP * 8));
-  v.ex_batch = exb;
   v.Xb = v.Pa = nullptr;
   v.slabs2 = nullptr;
   v.rowval = v.params = nullptr;

@@ -106,16 +106,15 @@ struct Plan {
   double* mfma64 = nullptr;    // MFMA-tiled Dr | D2r2 | D2s   (3 * NRP*NRP)
   float* mfma32 = nullptr;     // MFMA-tiled Dr | D2r2          (2 * NRP*NRP)
   double* vecs = nullptr;      // 8 vectors of length NRP (see VecId)
-  // implicit solves: quad-packed operator data (layout in sddc_solve.hip)
+  // implicit solves: operator data in MFMA fragment order (layout in sddc_frag.h)
   int NRS = 0;                 // nr rounded up to a multiple of 8
   int seg_m = 0, nseg = 0;     // rows per chain segment, segments per chain
   double* chain_L[3] = {nullptr, nullptr, nullptr};   // block inverses, K x NRP x NRS
-  double* chain_DL = nullptr;                         // D2 Linv_j of the A4 solve, per mode
   double* chain_D2 = nullptr;                         // D2 of the A4 solve (one block)
-  double* chain_Q[3] = {nullptr, nullptr, nullptr};   // row corrections (nseg > 1)
-  double* chain_E[3] = {nullptr, nullptr, nullptr};   // segment exit maps (nseg > 1)
-  double* chain_Lm[3] = {nullptr, nullptr, nullptr};  // MFMA-packed block inverses
-  double* chain_DLm = nullptr;                        // MFMA-packed D2 Linv_j (A4)
+  // the step's solves in the eigenbasis of the theta operator, when set
+  // (sddc_theta_solve.hip): W, V (sine, cosine; even, odd rows), U (sine), entry weights
+  double* theta = nullptr;
+  int theta_low[2] = {0, 0};   // psi rows per parity left to the chain: steps, sddc_bsub
   // NAB2 solves in the eigenbasis of r^2 - h r^2 Lap (fields 1, 2), when set:
   // per field lam [NRS] (padding 1), V [nr][NRS], V^-1 [NRS][NRS] (padding 0)
   int nab2_modal = 0;
@@ -133,9 +132,6 @@ struct Plan {
   void* F = nullptr;
   double* rowval = nullptr;
   double* params = nullptr;    // 2*max_batch: Ra, Ra_s staging
-  double* solve_scratch = nullptr;   // 4N + 256 doubles, sink of padded solve stores
-  double* chain_EX = nullptr;        // zero-entry segment exit states
-  int ex_batch = 0;                  // instances chain_EX holds
   int tune_solve_nbi = 0;            // instances per solve workgroup, 0 = automatic
   int tune_sub_batches = 1;          // parts of a batch on forked streams in graphs
   int tune_spectral_nb = 0;          // instances per spectral workgroup, 0 = automatic
@@ -181,6 +177,7 @@ int launch_rhs(const Plan& p, int B, const void* F, const double* L, int have_no
                double* G, hipStream_t s);
 int launch_solve(const Plan& p, int B, const double* G, double* Xout, double* Pout,
                  int fields_mask, int mask_out, hipStream_t s);
+int build_theta(Plan& p, const sddc_operators* ops);
 int build_chain(Plan& p, const sddc_operators* ops, int max_batch, int segment);
 void free_chain(Plan& p);
 int launch_mask(const Plan& p, int B, const double* X, double* out, hipStream_t s);

@@ -104,7 +104,8 @@ class Plan:
         return cls(_ops.build(N_fm, N_r, d, dt, Pr, Tau), symmetric, precision, max_batch, tuning)
 
     def tuning(self):
-        """Launch shapes in use: {'chain_segment': rows, 'solve_instances': n
+        """Launch shapes in use: {'chain_segment': N_fm/2 (chains) or less
+        (theta eigenbasis), 'solve_instances': shape of the chains' launch
         (0 = by batch), 'sub_batches': parts of a batch on forked streams in graphs,
         'nab2_solve': 1 per-mode block inverses, 2 eigenbasis,
         'spectral_instances': instances per spectral workgroup (0 = by batch)}."""

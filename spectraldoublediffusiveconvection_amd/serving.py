@@ -97,7 +97,7 @@ class Job:
 
 def class_bytes(N_fm, N_r, capacity, precision):
     """HBM footprint estimate of a time-integration class: operators and the
-    segment maps, plus per-slot state and workspace."""
+    solves' matrices, plus per-slot state and workspace."""
     nr = N_r - 1
     N = N_fm * nr
     rs = 4 if precision == "mixed" else 8
