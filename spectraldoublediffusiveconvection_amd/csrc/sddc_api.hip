@@ -451,21 +451,29 @@ int sddc_nlin_fx(sddc_plan* plan, int B, const double* X, double* out, void* str
   return SDDC_OK;
 }
 
-static int dfx_pipeline(Plan& p, int B, const double* dv, const double* X, const double* Ra,
-                        const double* Ras, bool linear_terms, double scale, double* out,
-                        hipStream_t s) {
+// The derivative of the nonlinear terms about X: the slabs of X, which stay for
+// any number of dv, ...
+static int dfx_point(Plan& p, int B, const double* X, hipStream_t s) {
   int rc;
-  const double *x = X, *v = dv;
+  const double* x = X;
   if (p.symmetric) {
     if ((rc = launch_mask(p, B, X, p.Xa, s))) return rc;
-    if ((rc = launch_mask(p, B, dv, p.Xb, s))) return rc;
     x = p.Xa;
-    v = p.Xb;
   }
   if ((rc = launch_suffix(p, B, x, p.P, s))) return rc;
-  if ((rc = launch_spectral(p, B, x, p.P, nullptr, nullptr, 0, nullptr, p.slabs, p.precision,
-                            nullptr, nullptr, s)))
-    return rc;
+  return launch_spectral(p, B, x, p.P, nullptr, nullptr, 0, nullptr, p.slabs, p.precision, nullptr,
+                         nullptr, s);
+}
+
+// ... and one dv.
+static int dfx_apply(Plan& p, int B, const double* dv, const double* Ra, const double* Ras,
+                     bool linear_terms, double scale, double* out, hipStream_t s) {
+  int rc;
+  const double* v = dv;
+  if (p.symmetric) {
+    if ((rc = launch_mask(p, B, dv, p.Xb, s))) return rc;
+    v = p.Xb;
+  }
   if ((rc = launch_suffix(p, B, v, p.Pa, s))) return rc;
   // the second slab set reuses slabs2 in the nonlinear pipeline precision
   if ((rc = launch_spectral(p, B, v, p.Pa, Ra, Ras, linear_terms ? 1 : 0, p.L, p.slabs2,
@@ -482,7 +490,8 @@ int sddc_nlin_dfx(sddc_plan* plan, int B, const double* dv, const double* X, dou
   int rc = check_batch(p, B);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  if ((rc = dfx_pipeline(p, B, dv, X, nullptr, nullptr, false, 1.0, out, s))) return rc;
+  if ((rc = dfx_point(p, B, X, s))) return rc;
+  if ((rc = dfx_apply(p, B, dv, nullptr, nullptr, false, 1.0, out, s))) return rc;
   if (p.symmetric) return launch_mask(p, B, out, out, s);
   return SDDC_OK;
 }
@@ -498,6 +507,25 @@ int sddc_bsub(sddc_plan* plan, int B, int field, const double* g, double* f, voi
   return launch_solve_ex(p, B, g, N, off, f, N, off, nullptr, 1 << field, false,
                          (hipStream_t)stream);
 }
+
+}  // extern "C"
+
+int sddc::linearise(sddc_plan* plan, int B, const double* X, hipStream_t s) {
+  if (!plan) return fail(SDDC_ERR_INVALID, "null plan");
+  if (int rc = check_batch(plan->p, B)) return rc;
+  return dfx_point(plan->p, B, X, s);
+}
+
+int sddc::linearised(sddc_plan* plan, int B, const double* Ra, const double* Ra_s,
+                     const double* dv, double* out, hipStream_t s) {
+  Plan& p = plan->p;
+  if (int rc = dfx_apply(p, B, dv, Ra, Ra_s, true, -1 * p.dt, p.G, s)) return rc;
+  Plan v = p;
+  v.slabs = p.slabs2;   // the solve's workspace: the slabs of X stay
+  return launch_solve(v, B, p.G, out, nullptr, 7, 0, s);
+}
+
+extern "C" {
 
 static int step_once(Plan& p, int B, const double* Ra, const double* Ras, const double* src,
                      double* dst, int linear, hipStream_t s) {
@@ -670,13 +698,8 @@ int sddc_step_static(sddc_plan* plan, int B, const double* Ra, const double* Ra_
 
 int sddc_step_linearized(sddc_plan* plan, int B, const double* Ra, const double* Ra_s,
                          const double* dv, const double* X, double* out, void* stream) {
-  if (!plan) return fail(SDDC_ERR_INVALID, "null plan");
-  Plan& p = plan->p;
-  int rc = check_batch(p, B);
-  if (rc) return rc;
-  hipStream_t s = (hipStream_t)stream;
-  if ((rc = dfx_pipeline(p, B, dv, X, Ra, Ra_s, true, -1 * p.dt, p.G, s))) return rc;
-  return launch_solve(p, B, p.G, out, nullptr, 7, 0, s);
+  if (int rc = linearise(plan, B, X, (hipStream_t)stream)) return rc;
+  return linearised(plan, B, Ra, Ra_s, dv, out, (hipStream_t)stream);
 }
 
 int sddc_diagnostics(sddc_plan* plan, int B, const double* X, double* out, void* stream) {

@@ -22,6 +22,8 @@
 
 #include "sddc.h"
 
+struct sddc_plan;
+
 namespace sddc {
 
 constexpr int kMaxRadices = 24;
@@ -187,6 +189,12 @@ int launch_ke_rows(const Plan& p, int B, const void* slabs64, double* rowval, hi
 int launch_diag_final(const Plan& p, int B, const double* X, const double* rowval,
                       double* out, hipStream_t s);
 int nonlinear_lds_bytes(const Plan& p, int precision, int dfx);
+// sddc_step_linearized in two parts, for many dv about one X: the transforms'
+// input of X in the plan's workspace, then one dv.  Between the two no other call may
+// use the plan.
+int linearise(sddc_plan* plan, int B, const double* X, hipStream_t s);
+int linearised(sddc_plan* plan, int B, const double* Ra, const double* Ra_s, const double* dv,
+               double* out, hipStream_t s);
 // Raise a kernel's dynamic-LDS limit to `bytes` (once per size increase).
 int ensure_dynamic_lds(const void* fn, size_t bytes, std::atomic<size_t>& current);
 

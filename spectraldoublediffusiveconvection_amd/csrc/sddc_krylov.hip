@@ -20,7 +20,7 @@
 #include <functional>
 #include <vector>
 
-#include "sddc_internal.h"
+#include "sddc_krylov.h"
 
 struct sddc_krylov {
   sddc_plan* plan = nullptr;
@@ -33,53 +33,22 @@ struct sddc_krylov {
   double* t = nullptr;     // n+1 step output / work
   double* c[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};   // n+1 each, continuation
   double* scal = nullptr;      // device scalars: 1, 0, Ra of the linearisation, a dot product
-  double* partial = nullptr;   // (m+2) x kBlocks partial sums
+  double* partial = nullptr;   // (m+2) x chunks partial dot products
+  double* npart = nullptr;     // updates: partial sums of a norm
   double* h = nullptr;         // 2(m+2)+1: first and second Gram-Schmidt projections, a norm
   // pinned host mirror (hipHostMalloc, 2(m+2)+4 doubles): projections, then
   // the scalar slot of norm2/get_scalar; every copy is an async DMA on the
   // caller's stream followed by a wait on that stream only
   double* hpin = nullptr;
+  hipEvent_t copied = nullptr;   // an Arnoldi step's projections are in hpin
 };
 
 namespace sddc {
 
-constexpr int kRedThreads = 256;
-constexpr int kBlocks = 240;   // workgroups of the reductions
+using krylov::Basis;
+using krylov::Gate;
 
-// partial[i][blk] = sum over this workgroup's chunk of A_i . x for i < nv,
-// where A_i = V + i*ld (or x itself when V is null: partial norm of x).
-__global__ __launch_bounds__(kRedThreads) void k_dots(const double* __restrict__ V,
-                                                      const double* __restrict__ x, int n,
-                                                      int ld, int nv,
-                                                      double* __restrict__ partial) {
-  __shared__ double red[kRedThreads];
-  const int chunk = (n + gridDim.x - 1) / gridDim.x;
-  const int e0 = blockIdx.x * chunk;
-  const int e1 = min(n, e0 + chunk);
-  for (int i = 0; i < nv; ++i) {
-    const double* a = V ? V + (size_t)i * ld : x;
-    double s = 0.0;
-    for (int e = e0 + threadIdx.x; e < e1; e += blockDim.x) s = fma(a[e], x[e], s);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int st = kRedThreads / 2; st > 0; st >>= 1) {
-      if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[(size_t)i * gridDim.x + blockIdx.x] = red[0];
-    __syncthreads();
-  }
-}
-
-// out[i] = (acc ? out[i] : 0) + sum_blk partial[i][blk], fixed order.
-__global__ void k_reduce(const double* __restrict__ partial, int nblk, int nv, int acc,
-                         double* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nv) return;
-  double s = 0.0;
-  for (int b = 0; b < nblk; ++b) s += partial[(size_t)i * nblk + b];
-  out[i] = acc ? out[i] + s : s;
-}
+constexpr Gate kNoGate{nullptr, -1};
 
 // y = alpha*y + beta * sum_{i<nv} c_i V_i   (c on the device, V_i = V + i*ld)
 __global__ void k_combine(double* __restrict__ y, const double* __restrict__ V,
@@ -113,16 +82,23 @@ static int axpby(double* z, const double* x, const double* y, int n, double a, d
 // aligned like the caller's states.
 static int basis_ld(int len) { return (len + 7) & ~7; }
 
-// out[0..nv) (device) = V_i . x over len entries (V_i = V + i*basis_ld(len)),
-// optionally accumulated
-static int dots(sddc_krylov& k, const double* V, const double* x, int len, int nv, int acc,
-                double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_dots, dim3(kBlocks), dim3(kRedThreads), 0, s, V, x, len, basis_ld(len), nv,
-                     k.partial);
-  if (int rc = hip_check(hipGetLastError(), "k_dots")) return rc;
-  hipLaunchKernelGGL(k_reduce, dim3((nv + 63) / 64), dim3(64), 0, s, k.partial, kBlocks, nv, acc,
-                     out);
-  return hip_check(hipGetLastError(), "k_reduce");
+// *out (device) = a . x over len entries; a null: x . x
+static int dot(sddc_krylov& k, const double* a, const double* x, int len, double* out,
+               hipStream_t s) {
+  if (int rc = krylov::launch_dots(Basis{a, 0}, x, nullptr, len, 1, k.m + 2, k.partial, 1, kNoGate,
+                                   s))
+    return rc;
+  return krylov::launch_total(k.partial, k.m + 2, len, 1, out, 1, 1, kNoGate, s);
+}
+
+// w *= 1 / ||w||; ||w||^2 to *norm2.  Grid: updates.
+__global__ __launch_bounds__(krylov::kThreads) void k_normalise(double* __restrict__ w, int n,
+                                                                const double* __restrict__ npart,
+                                                                double* __restrict__ norm2) {
+  __shared__ double tmp[krylov::kThreads / 64];
+  const double total = krylov::norm_total(npart, gridDim.x, tmp);
+  krylov::scale_update(w, n, sqrt(total));
+  if (blockIdx.x == 0 && threadIdx.x == 0) *norm2 = total;
 }
 
 static double* proj2(sddc_krylov& k) { return k.h + (k.m + 2); }
@@ -130,20 +106,22 @@ static double* norm_slot(sddc_krylov& k) { return k.h + 2 * (k.m + 2); }
 static double* host_scalar(sddc_krylov& k) { return k.hpin + 2 * (k.m + 2); }
 
 static int norm2(sddc_krylov& k, const double* x, int len, double* host, hipStream_t s) {
-  if (int rc = dots(k, nullptr, x, len, 1, 0, norm_slot(k), s)) return rc;
+  if (int rc = dot(k, nullptr, x, len, norm_slot(k), s)) return rc;
   SDDC_HIP(hipMemcpyAsync(host_scalar(k), norm_slot(k), sizeof(double), hipMemcpyDeviceToHost, s));
   SDDC_HIP(hipStreamSynchronize(s));
   *host = std::sqrt(*host_scalar(k));
   return SDDC_OK;
 }
 
-// Jacobian-vector product out = J v of F(X) = Step(X) - X.
+// Jacobian-vector product J v = out - *sub of F(X) = Step(X) - X (*sub: v, or
+// null).  The derivative needs X in the plan's workspace (linearise).
 static int jv(sddc_krylov& k, const double* Ra, const double* Ras, const double* X,
-              const double* v, double* out, int fd, hipStream_t s) {
+              const double* v, double* out, const double** sub, int fd, hipStream_t s) {
   int rc;
+  *sub = nullptr;
   if (!fd) {
-    if ((rc = sddc_step_linearized(k.plan, 1, Ra, Ras, v, X, out, s))) return rc;
-    return axpby(out, out, v, k.n, 1.0, -1.0, s);
+    *sub = v;
+    return linearised(k.plan, 1, Ra, Ras, v, out, s);
   }
   // finite difference of the step: (Step(X + eps v) - Step(X)) / eps - v,
   // Step(X) is kept in k.t by the caller
@@ -185,15 +163,17 @@ static int get_scalar(sddc_krylov& k, const double* x, double* host, hipStream_t
   return SDDC_OK;
 }
 
-// A linear operator out = A v on vectors of length len.
-using ApplyFn = std::function<int(const double* v, double* out)>;
+// A linear operator A v = out - *sub on vectors of length len (*sub may be null).
+using ApplyFn = std::function<int(const double* v, double* out, const double** sub)>;
 
 // Restarted GMRES(m) on A x = b (x holds the initial guess): CGS2 Arnoldi
 // on the basis V (row stride len), Givens rotations and the triangular solve
 // of the small least-squares problem on the host.  Stops at
-// ||b - A x|| <= max(atol, rtol ||b||).
-static int gmres_core(sddc_krylov& k, int len, const ApplyFn& A, const double* b, double* x,
-                      const sddc_krylov_opts& opts, sddc_krylov_info* info, hipStream_t s) {
+// ||b - A x|| <= max(atol, rtol ||b||).  ahead: the product of the next Arnoldi
+// step is queued before the host waits for this step's projections, so that the device
+// does not wait for the host; the last one of a cycle is then not used.
+static int gmres_core(sddc_krylov& k, int len, const ApplyFn& A, bool ahead, const double* b,
+                      double* x, const sddc_krylov_opts& opts, sddc_krylov_info* info, hipStream_t s) {
   const int m = k.m, ld = basis_ld(len);
   int rc, total = 0;
   double bnorm, rnorm = 0.0;
@@ -203,7 +183,9 @@ static int gmres_core(sddc_krylov& k, int len, const ApplyFn& A, const double* b
   int converged = 0, restarts = 0;
   for (; restarts < std::max(1, opts.max_restarts); ++restarts) {
     // r = b - A x
-    if ((rc = A(x, k.r))) return rc;
+    const double* sub;
+    if ((rc = A(x, k.r, &sub))) return rc;
+    if (sub && (rc = axpby(k.r, k.r, sub, len, 1.0, -1.0, s))) return rc;
     if ((rc = axpby(k.r, b, k.r, len, 1.0, -1.0, s))) return rc;
     double beta;
     if ((rc = norm2(k, k.r, len, &beta, s))) return rc;
@@ -219,25 +201,31 @@ static int gmres_core(sddc_krylov& k, int len, const ApplyFn& A, const double* b
     for (; j < m; ++j) {
       double* vj = k.V + (size_t)j * ld;
       double* vn = k.V + (size_t)(j + 1) * ld;
-      if ((rc = A(vj, vn))) return rc;
+      if ((j == 0 || !ahead) && (rc = A(vj, vn, &sub))) return rc;
       ++total;
       // CGS2: h = V^T w, w -= V h, twice (projections accumulated)
-      if ((rc = dots(k, k.V, vn, len, j + 1, 0, k.h, s))) return rc;
-      hipLaunchKernelGGL(k_combine, dim3(grid_for(len)), dim3(256), 0, s, vn, k.V, k.h, len, ld,
-                         j + 1, 1.0, -1.0);
-      if ((rc = hip_check(hipGetLastError(), "k_combine"))) return rc;
-      if ((rc = dots(k, k.V, vn, len, j + 1, 0, proj2(k), s))) return rc;
-      hipLaunchKernelGGL(k_combine, dim3(grid_for(len)), dim3(256), 0, s, vn, k.V, proj2(k), len,
-                         ld, j + 1, 1.0, -1.0);
-      if ((rc = hip_check(hipGetLastError(), "k_combine"))) return rc;
-      // both projection sets in one copy (h holds them back to back)
-      SDDC_HIP(hipMemcpyAsync(k.hpin, k.h, 2 * (size_t)(m + 2) * sizeof(double),
+      const Basis V{k.V, (size_t)ld};
+      for (int pass = 0; pass < 2; ++pass) {
+        const double* first = pass ? nullptr : sub;
+        if ((rc = krylov::launch_dots(V, vn, first, len, j + 1, m + 2, k.partial, 1, kNoGate, s)))
+          return rc;
+        if ((rc = krylov::launch_project(vn, V, first, len, j + 1, k.partial, m + 2,
+                                         pass ? proj2(k) : k.h, 0, pass ? k.npart : nullptr, 1,
+                                         kNoGate, s)))
+          return rc;
+      }
+      hipLaunchKernelGGL(k_normalise, dim3(krylov::updates(len)), dim3(krylov::kThreads), 0, s, vn,
+                         len, k.npart, norm_slot(k));
+      if ((rc = hip_check(hipGetLastError(), "k_normalise"))) return rc;
+      // both projection sets and the norm in one copy (they lie back to back)
+      SDDC_HIP(hipMemcpyAsync(k.hpin, k.h, (2 * (size_t)(m + 2) + 1) * sizeof(double),
                               hipMemcpyDeviceToHost, s));
-      double hn;
-      if ((rc = norm2(k, vn, len, &hn, s))) return rc;   // synchronises the copy too
+      SDDC_HIP(hipEventRecord(k.copied, s));
+      if (ahead && j + 1 < m && (rc = A(vn, vn + ld, &sub))) return rc;
+      SDDC_HIP(hipEventSynchronize(k.copied));
+      const double hn = std::sqrt(*host_scalar(k));
       for (int i = 0; i <= j; ++i) H[(size_t)i * m + j] = k.hpin[i] + k.hpin[(m + 2) + i];
       H[(size_t)(j + 1) * m + j] = hn;
-      if (hn > 0.0 && (rc = axpby(vn, vn, nullptr, len, 1.0 / hn, 0.0, s))) return rc;
       // Givens rotations of the new column
       for (int i = 0; i < j; ++i) {
         const double a = H[(size_t)i * m + j], c = H[(size_t)(i + 1) * m + j];
@@ -330,7 +318,10 @@ int sddc_krylov_create(sddc_plan* plan, int restart, sddc_krylov** out) {
   if (!rc) rc = A(&k->t, n1);
   for (int i = 0; i < 5 && !rc; ++i) rc = A(&k->c[i], n1);
   if (!rc) rc = A(&k->scal, 4);
-  if (!rc) rc = A(&k->partial, (size_t)(restart + 2) * kBlocks);
+  if (!rc) rc = A(&k->partial, (size_t)(restart + 2) * krylov::chunks(k->n + 1));
+  if (!rc) rc = A(&k->npart, krylov::updates(k->n + 1));
+  if (!rc)
+    rc = hip_check(hipEventCreateWithFlags(&k->copied, hipEventDisableTiming), "krylov event");
   if (!rc) rc = A(&k->h, 2 * ((size_t)restart + 2) + 1);
   if (!rc)
     rc = hip_check(hipHostMalloc((void**)&k->hpin, (2 * ((size_t)restart + 2) + 4) * sizeof(double),
@@ -355,9 +346,10 @@ int sddc_krylov_destroy(sddc_krylov* k) {
   if (!k) return SDDC_OK;
   std::lock_guard<std::recursive_mutex> lk(device_state_mutex());
   double* bufs[] = {k->V, k->w, k->r, k->f, k->t, k->c[0], k->c[1], k->c[2], k->c[3], k->c[4],
-                    k->scal, k->partial, k->h};
+                    k->scal, k->partial, k->npart, k->h};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
+  if (k->copied) (void)hipEventDestroy(k->copied);
   if (k->hpin) (void)hipHostFree(k->hpin);
   delete k;
   return SDDC_OK;
@@ -371,8 +363,11 @@ int sddc_gmres(sddc_krylov* k, const double* Ra, const double* Ra_s, const doubl
   const int fd = opts->finite_difference;
   int rc;
   if (fd && (rc = sddc_step(k->plan, 1, Ra, Ra_s, X, k->t, 1, 0, s))) return rc;
-  const ApplyFn J = [&](const double* v, double* out) { return jv(*k, Ra, Ra_s, X, v, out, fd, s); };
-  return gmres_core(*k, k->n, J, b, x, *opts, info, s);
+  if (!fd && (rc = linearise(k->plan, 1, X, s))) return rc;
+  const ApplyFn J = [&](const double* v, double* out, const double** sub) {
+    return jv(*k, Ra, Ra_s, X, v, out, sub, fd, s);
+  };
+  return gmres_core(*k, k->n, J, !fd, b, x, *opts, info, s);
 }
 
 int sddc_newton(sddc_krylov* k, const double* Ra, const double* Ra_s, double* X,
@@ -430,19 +425,23 @@ int sddc_arclength_step(sddc_krylov* k, const double* Ra_s, double* Y, double* Y
   double* Xc = k->c[3];     // masked state of the current corrector iteration
   double* dY = k->c[4];     // corrector update / predictor xi
   double* mu_c = k->scal + 2;   // Ra of the linearisation point (device)
-  double* dot = k->scal + 3;
+  double* xdot_v = k->scal + 3;
   *info = sddc_arclength_info{};
   int rc, krylov_total = 0;
   sddc_krylov_opts go = *opts;
 
   // Bordered operator DG(dY) at (Xc, mu_c) (Main.py:912-913)
   double mudot = 0.0;
-  const ApplyFn J = [&](const double* v, double* out) { return jv(*k, mu_c, Ra_s, Xc, v, out, fd, s); };
-  const ApplyFn DG = [&](const double* v, double* out) {
+  const ApplyFn J = [&](const double* v, double* out, const double** sub) {
+    return jv(*k, mu_c, Ra_s, Xc, v, out, sub, fd, s);
+  };
+  const ApplyFn DG = [&](const double* v, double* out, const double** sub) {
     int r;
-    if ((r = jv(*k, mu_c, Ra_s, Xc, v, out, fd, s))) return r;
-    if ((r = dots(*k, Xdot, v, n, 1, 0, dot, s))) return r;
-    hipLaunchKernelGGL(k_border, dim3(grid_for(n)), dim3(256), 0, s, out, v, dfmu, dot, n, delta,
+    if ((r = jv(*k, mu_c, Ra_s, Xc, v, out, sub, fd, s))) return r;
+    if (*sub && (r = axpby(out, out, *sub, n, 1.0, -1.0, s))) return r;
+    *sub = nullptr;
+    if ((r = dot(*k, Xdot, v, n, xdot_v, s))) return r;
+    hipLaunchKernelGGL(k_border, dim3(grid_for(n)), dim3(256), 0, s, out, v, dfmu, xdot_v, n, delta,
                        mudot);
     return hip_check(hipGetLastError(), "k_border");
   };
@@ -459,12 +458,13 @@ int sddc_arclength_step(sddc_krylov* k, const double* Ra_s, double* Y, double* Y
     if ((rc = pdfmu(*k, Xc, k->f, s))) return rc;
     if ((rc = axpby(k->f, k->f, nullptr, n, -1.0, 0.0, s))) return rc;
     if (fd && (rc = sddc_step(k->plan, 1, mu_c, Ra_s, Xc, k->t, 1, 0, s))) return rc;
+    if (!fd && (rc = linearise(k->plan, 1, Xc, s))) return rc;
     double bn;
     if ((rc = norm2(*k, k->f, n, &bn, s))) return rc;
     go.atol = tol * bn;   // atol = tol_newton ||b|| (Main.py:857)
     if ((rc = axpby(dY, dY, nullptr, n, 0.0, 0.0, s))) return rc;
     sddc_krylov_info gi{};
-    if ((rc = gmres_core(*k, n, J, k->f, dY, go, &gi, s))) return rc;
+    if ((rc = gmres_core(*k, n, J, !fd, k->f, dY, go, &gi, s))) return rc;
     krylov_total += gi.iterations;
     if (!gi.converged) {
       info->status = SDDC_ARC_PREDICTOR_FAILED;
@@ -512,18 +512,19 @@ int sddc_arclength_step(sddc_krylov* k, const double* Ra_s, double* Y, double* Y
     if ((rc = sddc_step(k->plan, 1, mu_c, Ra_s, Xc, k->t, 1, 0, s))) return rc;
     if ((rc = axpby(k->f, k->t, Xc, n, 1.0, -1.0, s))) return rc;
     if ((rc = axpby(k->r, Xc, X0, n, 1.0, -1.0, s))) return rc;
-    if ((rc = dots(*k, Xdot, k->r, n, 1, 0, dot, s))) return rc;
+    if ((rc = dot(*k, Xdot, k->r, n, xdot_v, s))) return rc;
     double xdot_dx, gx2;
-    if ((rc = get_scalar(*k, dot, &xdot_dx, s))) return rc;
+    if ((rc = get_scalar(*k, xdot_v, &xdot_dx, s))) return rc;
     const double gmu = delta * xdot_dx + (1.0 - delta) * mudot * (mu - mu0) - step;
     if ((rc = set_scalar(k->f + n, gmu, s))) return rc;
-    if ((rc = dots(*k, nullptr, k->f, n, 1, 0, dot, s))) return rc;
-    if ((rc = get_scalar(*k, dot, &gx2, s))) return rc;
+    if ((rc = dot(*k, nullptr, k->f, n, xdot_v, s))) return rc;
+    if ((rc = get_scalar(*k, xdot_v, &gx2, s))) return rc;
     const double bn = std::sqrt(delta * gx2 + (1.0 - delta) * gmu * gmu);
     go.atol = opts->tol_gmres * bn;   // Main.py:917-918
     if ((rc = axpby(dY, dY, nullptr, n + 1, 0.0, 0.0, s))) return rc;
+    if (!fd && (rc = linearise(k->plan, 1, Xc, s))) return rc;
     sddc_krylov_info gi{};
-    if ((rc = gmres_core(*k, n + 1, DG, k->f, dY, go, &gi, s))) return rc;
+    if ((rc = gmres_core(*k, n + 1, DG, !fd, k->f, dY, go, &gi, s))) return rc;
     krylov_total += gi.iterations;
     if ((rc = axpby(Y, Y, dY, n + 1, 1.0, -1.0, s))) return rc;
     if (!gi.converged) {
@@ -551,10 +552,11 @@ int sddc_arclength_step(sddc_krylov* k, const double* Ra_s, double* Y, double* Y
   // normalised in the weighted norm (Main.py:941-950)
   if ((rc = axpby(k->f, k->f, nullptr, n + 1, 0.0, 0.0, s))) return rc;
   if ((rc = set_scalar(k->f + n, 1.0, s))) return rc;
+  if (!fd && (rc = linearise(k->plan, 1, Xc, s))) return rc;
   go.atol = tol;   // tol_newton * ||e_last||
   if ((rc = axpby(Y_dot, Y_dot, nullptr, n + 1, 0.0, 0.0, s))) return rc;
   sddc_krylov_info gi{};
-  if ((rc = gmres_core(*k, n + 1, DG, k->f, Y_dot, go, &gi, s))) return rc;
+  if ((rc = gmres_core(*k, n + 1, DG, !fd, k->f, Y_dot, go, &gi, s))) return rc;
   krylov_total += gi.iterations;
   info->krylov_iterations = krylov_total;
   if (!gi.converged) {   // Main.py:943-944: a zero tangent
@@ -563,8 +565,8 @@ int sddc_arclength_step(sddc_krylov* k, const double* Ra_s, double* Y, double* Y
   }
   info->tangent_ok = 1;
   double t2, tmu;
-  if ((rc = dots(*k, nullptr, Y_dot, n, 1, 0, dot, s))) return rc;
-  if ((rc = get_scalar(*k, dot, &t2, s))) return rc;
+  if ((rc = dot(*k, nullptr, Y_dot, n, xdot_v, s))) return rc;
+  if ((rc = get_scalar(*k, xdot_v, &t2, s))) return rc;
   if ((rc = get_scalar(*k, Y_dot + n, &tmu, s))) return rc;
   const double scale = std::sqrt(delta * t2 + (1.0 - delta) * tmu * tmu);
   if ((rc = axpby(Y_dot, Y_dot, nullptr, n + 1, 1.0 / scale, 0.0, s))) return rc;

@@ -16,9 +16,8 @@
 // once per Newton iteration.  An instance that has converged is frozen (its
 // least-squares data and solution are no longer touched) while the others go
 // on, so its result does not depend on the other instances of the batch: the
-// dot products reduce over a fixed per-instance split into kBlocks partial
-// sums and a fixed-order sum, and the step kernels' launch shapes are the
-// plan's.  A batch of one is how a single job runs, so a job gives the same
+// dot products' partial sums and their order depend on the vector length alone,
+// and the step kernels' launch shapes are the plan's.  A batch of one is how a single job runs, so a job gives the same
 // bits alone and batched with others.
 //
 // Basis layout: V[j][b][n] (j = 0..m, b < capacity, n = 3N): the j-th basis
@@ -27,64 +26,27 @@
 #include <cmath>
 #include <vector>
 
-#include "sddc_internal.h"
+#include "sddc_krylov.h"
 
 namespace sddc {
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kBlocks = 240;   // partial sums per instance and dot product
+using krylov::Basis;
+using krylov::Gate;
+using krylov::kThreads;
 
 // per-instance scalars (double) and flags (int)
 enum Scal { S_NORM2 = 0, S_TARGET, S_INV, S_EPS, S_RES, S_XNORM2, S_VNORM2, S_ERR, S_BNORM, kNS };
+// (kNF is krylov::kFlags)
 enum Flag { F_ACTIVE = 0, F_GCONV, F_NEWTON, F_JEND, F_ITERS, F_CYCLE, F_RESTARTS, F_ZEROV, kNF };
 
 struct Ctx {
   int n, m, cap, B;
-  double *V, *F, *dv, *R, *T, *partial, *h, *h2, *H, *cs, *sn, *g, *y, *sc;
+  double *V, *F, *dv, *R, *T, *partial, *npart, *h, *h2, *H, *cs, *sn, *g, *y, *sc;
   int* fl;
+  Gate gate(int which) const { return Gate{fl, which}; }
 };
-
-// partial[b][i][blk] = (V_i[b] . x[b]) over this block's chunk, i < nv; V == null: x . x
-__global__ __launch_bounds__(kThreads) void k_bdots(const double* __restrict__ V, size_t strideJ,
-                                                    const double* __restrict__ x, int n, int nv,
-                                                    int pstride, double* __restrict__ partial,
-                                                    const int* __restrict__ fl, int gate) {
-  const int b = blockIdx.y;
-  if (gate >= 0 && !fl[(size_t)b * kNF + gate]) return;
-  __shared__ double red[kThreads];
-  const int chunk = (n + gridDim.x - 1) / gridDim.x;
-  const int e0 = blockIdx.x * chunk;
-  const int e1 = min(n, e0 + chunk);
-  const double* xb = x + (size_t)b * n;
-  for (int i = 0; i < nv; ++i) {
-    const double* a = V ? V + i * strideJ + (size_t)b * n : xb;
-    double s = 0.0;
-    for (int e = e0 + threadIdx.x; e < e1; e += blockDim.x) s = fma(a[e], xb[e], s);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int st = kThreads / 2; st > 0; st >>= 1) {
-      if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[((size_t)b * pstride + i) * gridDim.x + blockIdx.x] = red[0];
-    __syncthreads();
-  }
-}
-
-// out[b*ostride + i] = sum over blocks, fixed order
-__global__ void k_breduce(const double* __restrict__ partial, int pstride, int nv,
-                          double* __restrict__ out, int ostride, const int* __restrict__ fl,
-                          int gate) {
-  const int b = blockIdx.x;
-  if (gate >= 0 && !fl[(size_t)b * kNF + gate]) return;
-  for (int i = threadIdx.x; i < nv; i += blockDim.x) {
-    const double* p = partial + ((size_t)b * pstride + i) * kBlocks;
-    double s = 0.0;
-    for (int q = 0; q < kBlocks; ++q) s += p[q];
-    out[(size_t)b * ostride + i] = s;
-  }
-}
+static_assert(kNF == krylov::kFlags, "flags per instance");
 
 // y[b] = alpha y[b] + beta sum_{i < nv_b} c[b][i] V_i[b]  (nv_b = the instance's
 // F_JEND when nv < 0, else nv)
@@ -152,47 +114,64 @@ __global__ void k_cycle_start(double* __restrict__ sc, int* __restrict__ fl,
   f[F_JEND] = 0;
 }
 
-// Arnoldi step j of every active instance: Hessenberg column j from the two
-// projection sets and ||w||, the previous rotations, a new rotation, the
-// residual estimate |g_{j+1}|; inactive from now on when it is <= target or
-// w vanished.  S_INV gets 1/||w|| for the normalisation of the new vector.
-__global__ void k_givens(const double* __restrict__ h, const double* __restrict__ h2,
-                         double* __restrict__ H, double* __restrict__ cs, double* __restrict__ sn,
-                         double* __restrict__ g, double* __restrict__ sc, int* __restrict__ fl,
-                         int j, int m, int B) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  int* f = fl + (size_t)b * kNF;
-  if (!f[F_ACTIVE]) return;
-  double* s = sc + (size_t)b * kNS;
-  const double* hb = h + (size_t)b * (m + 2);
-  const double* h2b = h2 + (size_t)b * (m + 2);
+// Arnoldi step j of every active instance: w normalised (by all workgroups of
+// the instance; grid: updates, B), and in its first one the Hessenberg column j
+// from the two projection sets and ||w||, the previous rotations, a new rotation,
+// the residual estimate |g_{j+1}|; inactive from now on when it is <= target or w
+// vanished.  The flag that this changes is not read here: skipped instances are
+// those whose partial norms start with -1.  The rotations are a serial chain, so
+// the column and they are staged in LDS (3 (m + 2) doubles): with their loads in
+// the chain it took 10 us at 25 columns.
+__global__ __launch_bounds__(kThreads) void k_givens(
+    double* __restrict__ w, int n, const double* __restrict__ npart, const double* __restrict__ h,
+    const double* __restrict__ h2, double* __restrict__ H, double* __restrict__ cs,
+    double* __restrict__ sn, double* __restrict__ g, double* __restrict__ sc,
+    int* __restrict__ fl, int j, int m) {
+  extern __shared__ double col[];
+  __shared__ double tmp[kThreads / 64];
+  const int b = blockIdx.y;
+  npart += (size_t)b * gridDim.x;
+  if (npart[0] < 0.0) return;
+  const double hn = sqrt(krylov::norm_total(npart, gridDim.x, tmp));
+  krylov::scale_update(w + (size_t)b * n, n, hn);
+  if (blockIdx.x != 0) return;
+  double* lc = col + m + 2;
+  double* ls = lc + m + 2;
   double* Hb = H + (size_t)b * (m + 1) * m;
   double* csb = cs + (size_t)b * m;
   double* snb = sn + (size_t)b * m;
-  double* gb = g + (size_t)b * (m + 1);
-  const double hn = sqrt(s[S_NORM2]);
-  for (int i = 0; i <= j; ++i) Hb[(size_t)i * m + j] = hb[i] + h2b[i];
-  Hb[(size_t)(j + 1) * m + j] = hn;
-  for (int i = 0; i < j; ++i) {
-    const double a = Hb[(size_t)i * m + j], c = Hb[(size_t)(i + 1) * m + j];
-    Hb[(size_t)i * m + j] = csb[i] * a + snb[i] * c;
-    Hb[(size_t)(i + 1) * m + j] = -snb[i] * a + csb[i] * c;
+  for (int i = threadIdx.x; i <= j; i += kThreads) {
+    col[i] = h[(size_t)b * (m + 2) + i] + h2[(size_t)b * (m + 2) + i];
+    lc[i] = i < j ? csb[i] : 0.0;
+    ls[i] = i < j ? snb[i] : 0.0;
   }
-  const double a = Hb[(size_t)j * m + j], c = Hb[(size_t)(j + 1) * m + j];
-  const double den = hypot(a, c);
-  csb[j] = den > 0.0 ? a / den : 1.0;
-  snb[j] = den > 0.0 ? c / den : 0.0;
-  Hb[(size_t)j * m + j] = den;
-  Hb[(size_t)(j + 1) * m + j] = 0.0;
-  gb[j + 1] = -snb[j] * gb[j];
-  gb[j] = csb[j] * gb[j];
-  const double res = fabs(gb[j + 1]);
-  s[S_RES] = res;
-  s[S_INV] = hn > 0.0 ? 1.0 / hn : 0.0;
-  f[F_JEND] = j + 1;
-  f[F_ITERS] += 1;
-  if (res <= s[S_TARGET] || hn == 0.0) f[F_ACTIVE] = 0;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double a = col[0];
+    for (int i = 0; i < j; ++i) {
+      const double c = col[i + 1];
+      col[i] = lc[i] * a + ls[i] * c;
+      a = -ls[i] * a + lc[i] * c;
+    }
+    const double den = hypot(a, hn);
+    const double cj = den > 0.0 ? a / den : 1.0, sj = den > 0.0 ? hn / den : 0.0;
+    csb[j] = cj;
+    snb[j] = sj;
+    col[j] = den;
+    double* s = sc + (size_t)b * kNS;
+    int* f = fl + (size_t)b * kNF;
+    double* gb = g + (size_t)b * (m + 1);
+    const double gj = gb[j], res = fabs(sj * gj);
+    gb[j + 1] = -sj * gj;
+    gb[j] = cj * gj;
+    s[S_RES] = res;
+    f[F_JEND] = j + 1;
+    f[F_ITERS] += 1;
+    if (res <= s[S_TARGET] || hn == 0.0) f[F_ACTIVE] = 0;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i <= j; i += kThreads) Hb[(size_t)i * m + j] = col[i];
+  if (threadIdx.x == 0) Hb[(size_t)(j + 1) * m + j] = 0.0;
 }
 
 // End of a cycle: y = H(0:jend, 0:jend)^-1 g(0:jend) for instances that ran
@@ -274,14 +253,12 @@ __global__ void k_newton_err(double* __restrict__ sc, const int* __restrict__ fl
   s[S_ERR] = xn > 0.0 ? sqrt(s[S_VNORM2]) / xn : INFINITY;
 }
 
-// sc[b][slot] = sum over the fixed per-instance split of x[b] . x[b]
+// sc[b][slot] = x[b] . x[b]
 int norms2(Ctx& c, const double* x, int slot, int gate, hipStream_t s) {
-  hipLaunchKernelGGL(k_bdots, dim3(kBlocks, c.B), dim3(kThreads), 0, s, nullptr, (size_t)0, x,
-                     c.n, 1, c.m + 2, c.partial, c.fl, gate);
-  if (int rc = hip_check(hipGetLastError(), "k_bdots")) return rc;
-  hipLaunchKernelGGL(k_breduce, dim3(c.B), dim3(64), 0, s, c.partial, c.m + 2, 1, c.sc + slot,
-                     (int)kNS, c.fl, gate);
-  return hip_check(hipGetLastError(), "k_breduce");
+  if (int rc = krylov::launch_dots(Basis{nullptr, 0}, x, nullptr, c.n, 1, c.m + 2, c.partial, c.B,
+                                   c.gate(gate), s))
+    return rc;
+  return krylov::launch_total(c.partial, c.m + 2, c.n, 1, c.sc + slot, kNS, c.B, c.gate(gate), s);
 }
 
 int vgrid(int n) { return std::min(64, (n + kThreads - 1) / kThreads); }
@@ -302,7 +279,7 @@ struct sddc_newton_batch {
   sddc_plan* plan = nullptr;
   int n = 0, m = 0, cap = 0;
   double *V = nullptr, *F = nullptr, *dv = nullptr, *R = nullptr, *T = nullptr;
-  double *partial = nullptr, *h = nullptr, *h2 = nullptr, *H = nullptr, *cs = nullptr,
+  double *partial = nullptr, *npart = nullptr, *h = nullptr, *h2 = nullptr, *H = nullptr, *cs = nullptr,
          *sn = nullptr, *g = nullptr, *y = nullptr, *sc = nullptr;
   int* fl = nullptr;
   int* hfl = nullptr;       // pinned host copy of the flags
@@ -325,6 +302,7 @@ Ctx ctx_of(sddc_newton_batch* k, int B) {
   c.R = k->R;
   c.T = k->T;
   c.partial = k->partial;
+  c.npart = k->npart;
   c.h = k->h;
   c.h2 = k->h2;
   c.H = k->H;
@@ -337,13 +315,15 @@ Ctx ctx_of(sddc_newton_batch* k, int B) {
   return c;
 }
 
-// J v for every instance into out (B vectors of n)
+// J v = out - *sub for every instance (B vectors of n; *sub: v, or null).  The
+// derivative needs X in the plan's workspace (linearise).
 int jv(sddc_newton_batch* k, Ctx& c, const double* Ra, const double* Ras, const double* X,
-       const double* v, double* out, int fd, hipStream_t s) {
+       const double* v, double* out, const double** sub, int fd, hipStream_t s) {
   int rc;
+  *sub = nullptr;
   if (!fd) {
-    if ((rc = sddc_step_linearized(k->plan, c.B, Ra, Ras, v, X, out, s))) return rc;
-    return axpby(c, out, out, v, 1.0, -1.0, -1, s);
+    *sub = v;
+    return linearised(k->plan, c.B, Ra, Ras, v, out, s);
   }
   if ((rc = norms2(c, v, S_VNORM2, F_NEWTON, s))) return rc;
   hipLaunchKernelGGL(k_fd_point, dim3(vgrid(c.n), c.B), dim3(kThreads), 0, s, c.R, X, v, c.n,
@@ -373,13 +353,17 @@ int gmres(sddc_newton_batch* k, Ctx& c, const double* Ra, const double* Ras, con
           int fd, int max_restarts, int check_every, hipStream_t s) {
   const int m = c.m;
   const size_t sJ = (size_t)c.cap * c.n;   // stride between basis vectors j and j+1
+  const Basis V{c.V, sJ};
+  const double* sub;
   int rc;
+  if (!fd && (rc = linearise(k->plan, c.B, X, s))) return rc;
   for (int r = 0; r < std::max(1, max_restarts); ++r) {
     // r = F - J dv (with dv = 0 on the first cycle: r = F)
     if (r == 0) {
       if ((rc = axpby(c, c.V, c.F, nullptr, 1.0, 0.0, F_NEWTON, s))) return rc;
     } else {
-      if ((rc = jv(k, c, Ra, Ras, X, c.dv, c.V, fd, s))) return rc;
+      if ((rc = jv(k, c, Ra, Ras, X, c.dv, c.V, &sub, fd, s))) return rc;
+      if (sub && (rc = axpby(c, c.V, c.V, sub, 1.0, -1.0, F_NEWTON, s))) return rc;
       if ((rc = axpby(c, c.V, c.F, c.V, 1.0, -1.0, F_NEWTON, s))) return rc;
     }
     if ((rc = norms2(c, c.V, S_NORM2, F_NEWTON, s))) return rc;
@@ -394,29 +378,22 @@ int gmres(sddc_newton_batch* k, Ctx& c, const double* Ra, const double* Ras, con
     for (int j = 0; j < m; ++j) {
       double* vj = c.V + j * sJ;
       double* vn = c.V + (j + 1) * sJ;
-      if ((rc = jv(k, c, Ra, Ras, X, vj, vn, fd, s))) return rc;
+      if ((rc = jv(k, c, Ra, Ras, X, vj, vn, &sub, fd, s))) return rc;
       // CGS2 on the active instances: h = V^T w, w -= V h, twice
       for (int pass = 0; pass < 2; ++pass) {
-        double* hp = pass ? c.h2 : c.h;
-        hipLaunchKernelGGL(k_bdots, dim3(kBlocks, c.B), dim3(kThreads), 0, s, c.V, sJ, vn, c.n,
-                           j + 1, m + 2, c.partial, c.fl, (int)F_ACTIVE);
-        if ((rc = hip_check(hipGetLastError(), "k_bdots"))) return rc;
-        hipLaunchKernelGGL(k_breduce, dim3(c.B), dim3(64), 0, s, c.partial, m + 2, j + 1, hp,
-                           m + 2, c.fl, (int)F_ACTIVE);
-        if ((rc = hip_check(hipGetLastError(), "k_breduce"))) return rc;
-        hipLaunchKernelGGL(k_bcombine, dim3(vgrid(c.n), c.B), dim3(kThreads), 0, s, vn, c.V, sJ,
-                           hp, m + 2, j + 1, c.n, 1.0, -1.0, c.fl, (int)F_ACTIVE);
-        if ((rc = hip_check(hipGetLastError(), "k_bcombine"))) return rc;
+        const double* first = pass ? nullptr : sub;
+        if ((rc = krylov::launch_dots(V, vn, first, c.n, j + 1, m + 2, c.partial, c.B,
+                                      c.gate(F_ACTIVE), s)))
+          return rc;
+        if ((rc = krylov::launch_project(vn, V, first, c.n, j + 1, c.partial, m + 2,
+                                         pass ? c.h2 : c.h, m + 2, pass ? c.npart : nullptr, c.B,
+                                         c.gate(F_ACTIVE), s)))
+          return rc;
       }
-      if ((rc = norms2(c, vn, S_NORM2, F_ACTIVE, s))) return rc;
-      hipLaunchKernelGGL(k_givens, dim3(pgrid(c.B)), dim3(64), 0, s, c.h, c.h2, c.H, c.cs, c.sn,
-                         c.g, c.sc, c.fl, j, m, c.B);
+      hipLaunchKernelGGL(k_givens, dim3(krylov::updates(c.n), c.B), dim3(kThreads),
+                         3 * (m + 2) * sizeof(double), s, vn, c.n, c.npart, c.h, c.h2, c.H, c.cs,
+                         c.sn, c.g, c.sc, c.fl, j, m);
       if ((rc = hip_check(hipGetLastError(), "k_givens"))) return rc;
-      // normalise the new vector of the instances still iterating (an instance
-      // that converged at this step never reads it)
-      hipLaunchKernelGGL(k_bscale, dim3(vgrid(c.n), c.B), dim3(kThreads), 0, s, vn, c.n, c.sc,
-                         c.fl, (int)F_ACTIVE);
-      if ((rc = hip_check(hipGetLastError(), "k_bscale"))) return rc;
       if ((j + 1) % check_every == 0 || j + 1 == m) {
         if ((rc = read_flags(k, c.B, s))) return rc;
         if (!any_flag(k, c.B, F_ACTIVE)) break;
@@ -463,7 +440,8 @@ int sddc_newton_batch_create(sddc_plan* plan, int restart, int max_batch,
   if (!rc) rc = A(&k->dv, B * n);
   if (!rc) rc = A(&k->R, B * n);
   if (!rc) rc = A(&k->T, B * n);
-  if (!rc) rc = A(&k->partial, B * (m + 2) * kBlocks);
+  if (!rc) rc = A(&k->partial, B * (m + 2) * krylov::chunks(k->n));
+  if (!rc) rc = A(&k->npart, B * krylov::updates(k->n));
   if (!rc) rc = A(&k->h, B * (m + 2));
   if (!rc) rc = A(&k->h2, B * (m + 2));
   if (!rc) rc = A(&k->H, B * (m + 1) * m);
@@ -492,7 +470,7 @@ int sddc_newton_batch_create(sddc_plan* plan, int restart, int max_batch,
 int sddc_newton_batch_destroy(sddc_newton_batch* k) {
   if (!k) return SDDC_OK;
   std::lock_guard<std::recursive_mutex> lk(device_state_mutex());
-  double* bufs[] = {k->V, k->F, k->dv, k->R, k->T, k->partial, k->h, k->h2, k->H, k->cs,
+  double* bufs[] = {k->V, k->F, k->dv, k->R, k->T, k->partial, k->npart, k->h, k->h2, k->H, k->cs,
                     k->sn, k->g, k->y, k->sc};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
