@@ -486,6 +486,67 @@ __device__ void fft_run_ip(cplx<R>* buf, const FftShape& sh, const cplx<R>* __re
 }
 
 // ---------------------------------------------------------------------------
+// The in-place transform of any length up to 64 NC with factors 2, 3, 4 and 5:
+// chunk counts fixed by NC, the schedule make_shape's, the twiddles in the
+// per-pass layout (ip_twiddle_offset) in LDS.
+// ---------------------------------------------------------------------------
+template <typename R, int NC, int RADIX>
+__device__ __forceinline__ void fft_pass_nc(cplx<R>* buf, int L, int Ns,
+                                            const cplx<R>* __restrict__ tw, bool inv, int lane) {
+  constexpr int U = (NC + RADIX - 1) / RADIX;   // chunks of 64 butterflies
+  const int nb = L / RADIX;
+  const float rns = 1.0f / (float)Ns;
+  cplx<R> v[U][RADIX], w[U][RADIX];
+  int base[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int jr = lane + 64 * u;
+    const int j = jr < nb ? jr : nb - 1;
+    const int jq = qdiv(j, Ns, rns);
+    const int k = j - jq * Ns;
+    base[u] = jq * Ns * RADIX + k;
+#pragma unroll
+    for (int s = 0; s < RADIX; ++s) v[u][s] = buf[j + s * nb];
+#pragma unroll
+    for (int s = 1; s < RADIX; ++s) w[u][s] = tw_get(tw, (s - 1) * Ns + k, inv);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int s = 1; s < RADIX; ++s) v[u][s] = cmul(v[u][s], w[u][s]);
+    if (RADIX == 2) dft2(v[u]);
+    if (RADIX == 3) dft3(v[u], inv);
+    if (RADIX == 4) dft4(v[u], inv);
+    if (RADIX == 5) dft5(v[u], inv);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (lane + 64 * u < nb)
+#pragma unroll
+      for (int s = 0; s < RADIX; ++s) buf[base[u] + s * Ns] = v[u][s];
+}
+
+template <typename R, int NC>
+__device__ __forceinline__ void fft_run_nc(cplx<R>* buf, const FftShape& sh,
+                                           const cplx<R>* __restrict__ tw, bool inv, int lane) {
+  int Ns = 1;
+  for (int p = 0; p < sh.npass; ++p) {
+    const int r = sh.radix[p];
+    if (r == 4)
+      fft_pass_nc<R, NC, 4>(buf, sh.L, Ns, tw, inv, lane);
+    else if (r == 2)
+      fft_pass_nc<R, NC, 2>(buf, sh.L, Ns, tw, inv, lane);
+    else if (r == 3)
+      fft_pass_nc<R, NC, 3>(buf, sh.L, Ns, tw, inv, lane);
+    else
+      fft_pass_nc<R, NC, 5>(buf, sh.L, Ns, tw, inv, lane);
+    wave_lds_sync();
+    tw += (r - 1) * Ns;
+    Ns *= r;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // The in-place transform with the length a compile-time constant: the pass
 // schedule is make_shape's (radix 4 first, then 2, 3, 5), and every stride,
 // chunk count and quotient of a pass folds into the instruction stream.

@@ -216,11 +216,10 @@ __device__ __forceinline__ void scale_products(cplx<R>* O, int L, int* red, R (&
   __syncthreads();
 }
 
-// Threads of the generic kernel.  It only runs the linearised products of
-// grids shorter than 192 points (N_fm below 128; the longer grids have the
-// in-place kernels), so four wavefronts cover every loop over the grid, and
-// at 1024 threads its scale arrays spilled to scratch (the 128-VGPR limit of
-// four wavefronts per SIMD).
+// Threads of the generic kernel.  It runs the linearised products of mixed plans
+// and of grids that the in-place kernels do not take.  Four wavefronts: at 1024
+// threads its scale arrays spilled to scratch (the 128-VGPR limit of four
+// wavefronts per SIMD).
 constexpr int kNlGenericThreads = 256;
 
 template <typename R, bool DFX>
@@ -964,6 +963,306 @@ __global__ __launch_bounds__(640) void k_nonlinear_dfx_ip(FftShape sh,
                                 lane);
 }
 
+// ---------------------------------------------------------------------------
+// The in-place kernels for the other lengths L = 3K/2 <= 64 NC with factors 2, 3
+// and 5: ip_pack_pair, the products and ip_forward_project with the last column
+// partly filled and the mirrored coefficients read through LDS.  A workgroup is
+// bound by the latency of its passes; the general kernels (k_nonlinear_w,
+// k_nonlinear), which loop over chunks of a length known at run time, took
+// 13.3 us (F(X, X), K = 64, N_r = 20; 8.0 here) and 33 us (the derivative, K = 64,
+// N_r = 24; 9.2); 48 instances, N_r = 30, float64: K = 64 41.7 -> 19.4, 300 117 -> 68,
+// 540 198 -> 144 us, mixed: K = 90 25.8 -> 13.6, 300 47.7 -> 43.1.
+// ---------------------------------------------------------------------------
+template <typename R, int NC>
+__device__ __forceinline__ void nc_pack_pair(const SlabRows<R>& sg, int p, cplx<R>* A,
+                                             const cplx<R>* __restrict__ rot_g, R* sinv, int K,
+                                             int L, int lane) {
+  constexpr int NK = (2 * NC + 2) / 3;
+  using C = cplx<R>;
+  const R *u, *v = nullptr;
+  bool us, vs = false;
+  int um, vm = 0;
+  field_src(sg, 2 * p, u, us, um);
+  if (p < 4) field_src(sg, 2 * p + 1, v, vs, vm);
+  C rr[NC];
+  R du[NK], dv[NK];
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    const int k = lane + 64 * j < K ? lane + 64 * j : K - 1;
+    du[j] = u[k];
+    dv[j] = v ? v[k] : (R)0;
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) rr[c] = rot_g[lane + 64 * c < L ? lane + 64 * c : L - 1];
+  int eu = -1000, ev = -1000;
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    const int k = lane + 64 * j;
+    R a = du[j], c = dv[j];
+    if (um == 1) a = (R)k * a;
+    if (um == 2) a = (R)(-k) * a;
+    if (vm == 1) c = (R)k * c;
+    if (vm == 2) c = (R)(-k) * c;
+    if (k >= K) a = c = (R)0;
+    if (!(us && k == 0)) eu = max(eu, bexp(a));
+    if (!(vs && k == 0)) ev = max(ev, bexp(c));
+    du[j] = a;
+    dv[j] = c;
+  }
+  eu = __ockl_wfred_max_i32(eu);
+  ev = __ockl_wfred_max_i32(ev);
+  const R su = pow2_scale_e<R>(eu), sv = pow2_scale_e<R>(ev);
+  if (lane == 0) {
+    sinv[0] = (R)1 / su;
+    if (p < 4) sinv[1] = (R)1 / sv;
+  }
+  // scaled coefficients at mode k (a sine row's index 0 is never used), also
+  // staged in the pair's buffer: K pairs of reals in L complex values
+  R* cu = reinterpret_cast<R*>(A);
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    const int k = lane + 64 * j;
+    du[j] = su * (k == 0 ? (us ? (R)0 : du[j]) : (R)0.5 * du[j]);
+    dv[j] = sv * (k == 0 ? (vs ? (R)0 : dv[j]) : (R)0.5 * dv[j]);
+    if (k < K) {
+      cu[k] = du[j];
+      cu[K + k] = dv[j];
+    }
+  }
+  wave_lds_sync();
+  R mu[NC], mv[NC];   // mirrored: index L - k
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int m = L - (lane + 64 * c);
+    const bool in = m > 0 && m < K;
+    mu[c] = cu[in ? m : 0];
+    mv[c] = cu[K + (in ? m : 0)];
+    if (!in) mu[c] = mv[c] = (R)0;
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int k = lane + 64 * c;
+    const R dcu = c < NK ? du[c < NK ? c : 0] : (R)0;
+    const R dcv = c < NK ? dv[c < NK ? c : 0] : (R)0;
+    const R au = us ? mu[c] : dcu, av = vs ? mv[c] : dcv;
+    const R aum = k ? (us ? dcu : mu[c]) : (R)0;
+    const R avm = k ? (vs ? dcv : mv[c]) : (R)0;
+    if (k < L) A[k] = cmul(C{au + avm, av - aum}, rr[c]);
+  }
+}
+
+template <typename R, int NC>
+__device__ __forceinline__ void nc_forward_project(cplx<R> (&o)[NC], cplx<R>* O, int p,
+                                                   const cplx<R>* tw, const FftShape& sh,
+                                                   const cplx<R>* __restrict__ rot_g,
+                                                   R* __restrict__ F, int b, int i, int nr, int K,
+                                                   int lane) {
+  constexpr int NK = (2 * NC + 2) / 3;
+  using C = cplx<R>;
+  const int L = sh.L;
+  C er[NK];
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    const int k = lane + 64 * j < K ? lane + 64 * j : K - 1;
+    const int ka = (p == 0) ? L - k : k;   // sine coefficients read index L-k
+    er[j] = rot_g[ka < L ? ka : ka - L];
+  }
+  int e0 = -1000, e1 = -1000;
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    if (lane + 64 * c < L) {
+      e0 = max(e0, bexp(o[c].x));
+      e1 = max(e1, bexp(o[c].y));
+    }
+  e0 = __ockl_wfred_max_i32(e0);
+  e1 = __ockl_wfred_max_i32(e1);
+  const R s0 = pow2_scale_e<R>(e0), s1 = pow2_scale_e<R>(e1);
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    if (lane + 64 * c < L) O[lane + 64 * c] = {o[c].x * s0, o[c].y * s1};
+  wave_lds_sync();
+  fft_run_nc<R, NC>(O, sh, tw, false, lane);
+  const R i0 = (R)1 / s0, i1 = (R)1 / s1, invL = (R)1 / (R)L;
+  R* f0 = F + ((size_t)(b * 4 + 2 * p) * nr + i) * K;
+  R* f1 = F + ((size_t)(b * 4 + 2 * p + 1) * nr + i) * K;
+  C za[NK], zb[NK];
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    const int k = lane + 64 * j < K ? lane + 64 * j : K - 1;
+    const int ka = (p == 0) ? L - k : k;
+    za[j] = O[ka < L ? ka : ka - L];
+    zb[j] = O[(L - ka) < L ? L - ka : L - ka - L];
+  }
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    const int k = lane + 64 * j;
+    // X = (a + conj b)/2, Y = (a - conj b)/(2i); C = Re(conj(e) X), Re(conj(e) Y)
+    const R xr = (R)0.5 * (za[j].x + zb[j].x), xi = (R)0.5 * (za[j].y - zb[j].y);
+    const R yr = (R)0.5 * (za[j].y + zb[j].y), yi = (R)-0.5 * (za[j].x - zb[j].x);
+    const R c1 = er[j].x * xr + er[j].y * xi;
+    const R c2 = er[j].x * yr + er[j].y * yi;
+    R a1, a2;
+    if (p == 0) {   // sine coefficients (k = 0 is zero)
+      a1 = k > 0 ? ((R)2 * (c1 * i0)) * invL : (R)0;
+      a2 = k > 0 ? ((R)2 * (c2 * i1)) * invL : (R)0;
+    } else {        // cosine coefficients
+      a1 = ((R)2 * (c1 * i0)) * invL;
+      a2 = ((R)2 * (c2 * i1)) * invL;
+      if (k == 0) {
+        a1 *= (R)0.5;
+        a2 *= (R)0.5;
+      }
+    }
+    if (k < K) {
+      f0[k] = a1;
+      f1[k] = a2;
+    }
+  }
+}
+
+// Wavefront q < 5 synthesises pair q of X, q >= 5 (the derivative) pair q - 5 of
+// dv; wavefronts 0 and 1 form the products and reuse pair buffers 3 and 4.  LDS:
+// twiddles (L), the pair buffers (5 L or 10 L).
+template <typename R, int NC, bool DFX>
+__global__ __launch_bounds__(DFX ? 640 : 320) void k_nonlinear_nc(
+    FftShape sh, const cplx<R>* __restrict__ tw_g, const cplx<R>* __restrict__ rot_g, int K,
+    int nr, const R* __restrict__ slabs, const R* __restrict__ slabs2, R* __restrict__ F) {
+  constexpr int NTHR = DFX ? 640 : 320;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ R sinv[20];   // unscaling factors: fields of X, then of dv
+  using C = cplx<R>;
+  const int L = sh.L;
+  C* tw = reinterpret_cast<C*>(smem_raw);
+  C* buf = tw + L;
+  const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int i = blockIdx.x, b = blockIdx.y, p = q < 5 ? q : q - 5;
+  constexpr int NT = (64 * NC + NTHR - 1) / NTHR;
+  C twr[NT];   // in flight with the slab loads
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int k = threadIdx.x + NTHR * j;
+    twr[j] = tw_g[k < L ? k : L - 1];
+  }
+  const SlabRows<R> sg = slab_rows<R>(q < 5 ? slabs : slabs2, b, i, nr, K);
+  C* A = buf + (size_t)q * L;
+  nc_pack_pair<R, NC>(sg, p, A, rot_g, sinv + (q < 5 ? 0 : 10) + 2 * p, K, L, lane);
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    if (threadIdx.x + NTHR * j < L) tw[threadIdx.x + NTHR * j] = twr[j];
+  __syncthreads();   // twiddles in LDS
+  fft_run_nc<R, NC>(A, sh, tw, true, lane);
+  __syncthreads();
+
+  R is[9], id[9];
+#pragma unroll
+  for (int f = 0; f < 9; ++f) {
+    is[f] = sinv[f];
+    id[f] = DFX ? sinv[10 + f] : (R)0;
+  }
+  C o[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    if (q >= 2) break;
+    const int x = lane + 64 * c, qq = x < L ? x : L - 1;
+    const R gs = (R)grid_sign(qq, L);
+    const C w0 = buf[qq], w1 = buf[L + qq], w2 = buf[2 * L + qq];
+    const R JT = w0.x * is[0], Om = gs * w0.y * is[1];
+    const R kOm = w1.x * is[2], Dpsi = gs * w1.y * is[3];
+    if constexpr (!DFX) {
+      if (q == 0) {
+        // Matrix_Operators.py:791 (Dr applied to JT*omega after projection)
+        const R kDpsi = w2.x * is[4];
+        o[c] = {gs * (JT * Om), gs * (kDpsi * Om + Dpsi * kOm)};
+      } else {
+        // Matrix_Operators.py:792-793
+        const C w3 = buf[3 * L + qq], w4 = buf[4 * L + qq];
+        const R kT = gs * w2.y * is[5], DT = w3.x * is[6], kC = gs * w3.y * is[7],
+                DC = w4.x * is[8];
+        o[c] = {JT * DT - Dpsi * kT, JT * DC - Dpsi * kC};
+      }
+    } else {
+      // Frechet derivative (Matrix_Operators.py:884-887), as in k_nonlinear_dfx_ip
+      const C v0 = buf[5 * L + qq], v1 = buf[6 * L + qq], v2 = buf[7 * L + qq];
+      const R dJT = v0.x * id[0], dOm = gs * v0.y * id[1];
+      const R dkOm = v1.x * id[2], dDpsi = gs * v1.y * id[3];
+      const R dkDpsi = v2.x * id[4];
+      if (q == 0) {
+        const R kDpsi = w2.x * is[4];
+        R zx = JT * dOm + dJT * Om;
+        R zy = kDpsi * dOm;
+        zy += Dpsi * dkOm + dDpsi * kOm;
+        zy += dkDpsi * Om;
+        o[c] = {gs * zx, gs * zy};
+      } else {
+        const C w3 = buf[3 * L + qq], w4 = buf[4 * L + qq];
+        const C v3 = buf[8 * L + qq], v4 = buf[9 * L + qq];
+        const R kT = gs * w2.y * is[5], DT = w3.x * is[6], kC = gs * w3.y * is[7],
+                DC = w4.x * is[8];
+        const R dkT = gs * v2.y * id[5], dDT = v3.x * id[6], dkC = gs * v3.y * id[7],
+                dDC = v4.x * id[8];
+        R tx = dJT * DT, ty = dJT * DC;
+        tx -= dDpsi * kT;
+        ty -= dDpsi * kC;
+        tx -= Dpsi * dkT;
+        tx += JT * dDT;
+        ty -= Dpsi * dkC;
+        ty += JT * dDC;
+        o[c] = {tx, ty};
+      }
+    }
+  }
+  __syncthreads();   // every read of the pair buffers is done
+  if (q >= 2) return;
+  nc_forward_project<R, NC>(o, buf + (size_t)(3 + q) * L, q, tw, sh, rot_g, F, b, i, nr, K, lane);
+}
+
+template <typename R, int NC, bool DFX>
+static int launch_nl_nc(const Plan& p, int B, const void* slabs, const void* slabs2, void* F,
+                        hipStream_t s, const cplx<R>* tw, const cplx<R>* rot) {
+  const size_t lds = (DFX ? 11 : 6) * (size_t)p.M * sizeof(cplx<R>);
+  static std::atomic<size_t> cur{0};
+  if (int rc = ensure_dynamic_lds((const void*)k_nonlinear_nc<R, NC, DFX>, lds, cur)) return rc;
+  hipLaunchKernelGGL((k_nonlinear_nc<R, NC, DFX>), dim3(p.nr, B), dim3(DFX ? 640 : 320), lds, s,
+                     p.tabM.shape, tw, rot, p.K, p.nr, (const R*)slabs, (const R*)slabs2, (R*)F);
+  return hip_check(hipGetLastError(), "k_nonlinear_nc");
+}
+
+// Whether k_nonlinear_nc takes the plan's grid: no factor above 5 (its twiddle
+// layout), 3K = 2L, and at most 13 columns in float64.  In float, F(X, X) up to 8
+// columns, whose instances (3 columns for fewer) give the bits of k_nonlinear_w;
+// the others and the derivative differ from the general kernels in which product
+// of a sum the compiler fuses, 1e-7 relative, which mixed-precision runs would
+// show.
+template <typename R, bool DFX>
+static bool nl_nc_fits(const Plan& p) {
+  constexpr bool F64 = std::is_same<R, double>::value;
+  const FftShape& sh = p.tabM.shape;
+  for (int q = 0; q < sh.npass; ++q)
+    if (sh.radix[q] > 5) return false;
+  return sh.npass > 0 && 3 * p.K == 2 * sh.L && sh.L <= (F64 ? 64 * 13 : DFX ? 0 : 64 * 8) &&
+         (DFX ? 11 : 6) * (size_t)p.M * sizeof(cplx<R>) + 512 <= 160 * 1024;
+}
+
+template <typename R, bool DFX>
+static int dispatch_nl_nc(const Plan& p, int B, const void* slabs, const void* slabs2, void* F,
+                          hipStream_t s, const cplx<R>* tw, const cplx<R>* rot) {
+  const int nc = (p.M + 63) / 64;
+  if constexpr (std::is_same<R, double>::value) {
+    if (nc <= 1) return launch_nl_nc<R, 1, DFX>(p, B, slabs, slabs2, F, s, tw, rot);
+    if (nc <= 2) return launch_nl_nc<R, 2, DFX>(p, B, slabs, slabs2, F, s, tw, rot);
+    if (nc > 10) return launch_nl_nc<R, 13, DFX>(p, B, slabs, slabs2, F, s, tw, rot);
+    if (nc > 8) return launch_nl_nc<R, 10, DFX>(p, B, slabs, slabs2, F, s, tw, rot);
+  }
+  if constexpr (std::is_same<R, double>::value || !DFX) {
+    if (nc <= 3) return launch_nl_nc<R, 3, DFX>(p, B, slabs, slabs2, F, s, tw, rot);
+    if (nc <= 4) return launch_nl_nc<R, 4, DFX>(p, B, slabs, slabs2, F, s, tw, rot);
+    if (nc <= 6) return launch_nl_nc<R, 6, DFX>(p, B, slabs, slabs2, F, s, tw, rot);
+    if (nc <= 8) return launch_nl_nc<R, 8, DFX>(p, B, slabs, slabs2, F, s, tw, rot);
+  }
+  return fail(SDDC_ERR_UNSUPPORTED, "grid length outside the in-place kernels");
+}
+
 // Columns per lane NC of the in-place kernel for this plan, 0 when its
 // grid does not fit it (k_nonlinear_w is used then).
 static int nl_inplace_nc(const Plan& p) {
@@ -1046,6 +1345,7 @@ static int launch_nl_t(const Plan& p, int B, const void* slabs, const void* slab
       case 12: return launch_nl_ip<R, 12>(p, B, slabs, F, s, twp, rot);
       default: break;
     }
+    if (nl_nc_fits<R, false>(p)) return dispatch_nl_nc<R, false>(p, B, slabs, slabs2, F, s, twp, rot);
     if (lds + 64 > 160 * 1024)
       return fail(SDDC_ERR_UNSUPPORTED, "N_fm too large for the LDS nonlinear kernel");
     static std::atomic<size_t> curw{0};
@@ -1060,6 +1360,7 @@ static int launch_nl_t(const Plan& p, int B, const void* slabs, const void* slab
     case 12: return launch_nl_dfx_ip<R, 12>(p, B, slabs, slabs2, F, s, twp, rot);
     default: break;
   }
+  if (nl_nc_fits<R, true>(p)) return dispatch_nl_nc<R, true>(p, B, slabs, slabs2, F, s, twp, rot);
   if (lds + 16 * 18 * sizeof(int) > 160 * 1024)
     return fail(SDDC_ERR_UNSUPPORTED, "N_fm too large for the LDS nonlinear kernel");
   static std::atomic<size_t> cur{0};
