@@ -396,15 +396,11 @@ int sddc_transform(int kind, const double* in, double* out, int rows, int len_in
   return launch_transform(*t, kind, rows, len_in, n_out, in, out, (hipStream_t)stream);
 }
 
-static int prep_input(Plan& p, int B, const double* X, const double** use, hipStream_t s,
-                      double* scratch) {
-  *use = X;
-  if (p.symmetric) {
-    int rc = launch_mask(p, B, X, scratch, s);
-    if (rc) return rc;
-    *use = scratch;
-  }
-  return SDDC_OK;
+// The state a plan works on and its suffix sums: X, or its masked copy in scratch.
+static int prep_state(Plan& p, int B, const double* X, double* scratch, double* P,
+                      const double** use, hipStream_t s) {
+  *use = p.symmetric ? scratch : X;
+  return launch_suffix(p, B, X, P, p.symmetric ? scratch : nullptr, s);
 }
 
 int sddc_theta_ops(sddc_plan* plan, int B, const double* X, double* out, void* stream) {
@@ -414,8 +410,7 @@ int sddc_theta_ops(sddc_plan* plan, int B, const double* X, double* out, void* s
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   const double* x;
-  if ((rc = prep_input(p, B, X, &x, s, p.Xa))) return rc;
-  if ((rc = launch_suffix(p, B, x, p.P, s))) return rc;
+  if ((rc = prep_state(p, B, X, p.Xa, p.P, &x, s))) return rc;
   return launch_spectral(p, B, x, p.P, nullptr, nullptr, 0, nullptr, nullptr, SDDC_FP64, out,
                          nullptr, s);
 }
@@ -427,8 +422,7 @@ int sddc_derivatives(sddc_plan* plan, int B, const double* X, double* out, void*
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   const double* x;
-  if ((rc = prep_input(p, B, X, &x, s, p.Xa))) return rc;
-  if ((rc = launch_suffix(p, B, x, p.P, s))) return rc;
+  if ((rc = prep_state(p, B, X, p.Xa, p.P, &x, s))) return rc;
   return launch_spectral(p, B, x, p.P, nullptr, nullptr, 0, nullptr, nullptr, SDDC_FP64, nullptr,
                          out, s);
 }
@@ -440,8 +434,7 @@ int sddc_nlin_fx(sddc_plan* plan, int B, const double* X, double* out, void* str
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   const double* x;
-  if ((rc = prep_input(p, B, X, &x, s, p.Xa))) return rc;
-  if ((rc = launch_suffix(p, B, x, p.P, s))) return rc;
+  if ((rc = prep_state(p, B, X, p.Xa, p.P, &x, s))) return rc;
   if ((rc = launch_spectral(p, B, x, p.P, nullptr, nullptr, 0, nullptr, p.slabs, p.precision,
                             nullptr, nullptr, s)))
     return rc;
@@ -455,12 +448,8 @@ int sddc_nlin_fx(sddc_plan* plan, int B, const double* X, double* out, void* str
 // any number of dv, ...
 static int dfx_point(Plan& p, int B, const double* X, hipStream_t s) {
   int rc;
-  const double* x = X;
-  if (p.symmetric) {
-    if ((rc = launch_mask(p, B, X, p.Xa, s))) return rc;
-    x = p.Xa;
-  }
-  if ((rc = launch_suffix(p, B, x, p.P, s))) return rc;
+  const double* x;
+  if ((rc = prep_state(p, B, X, p.Xa, p.P, &x, s))) return rc;
   return launch_spectral(p, B, x, p.P, nullptr, nullptr, 0, nullptr, p.slabs, p.precision, nullptr,
                          nullptr, s);
 }
@@ -469,12 +458,8 @@ static int dfx_point(Plan& p, int B, const double* X, hipStream_t s) {
 static int dfx_apply(Plan& p, int B, const double* dv, const double* Ra, const double* Ras,
                      bool linear_terms, double scale, double* out, hipStream_t s) {
   int rc;
-  const double* v = dv;
-  if (p.symmetric) {
-    if ((rc = launch_mask(p, B, dv, p.Xb, s))) return rc;
-    v = p.Xb;
-  }
-  if ((rc = launch_suffix(p, B, v, p.Pa, s))) return rc;
+  const double* v;
+  if ((rc = prep_state(p, B, dv, p.Xb, p.Pa, &v, s))) return rc;
   // the second slab set reuses slabs2 in the nonlinear pipeline precision
   if ((rc = launch_spectral(p, B, v, p.Pa, Ra, Ras, linear_terms ? 1 : 0, p.L, p.slabs2,
                             p.precision, nullptr, nullptr, s)))
@@ -548,8 +533,7 @@ static int run_steps(Plan& p, int B, const double* Ra, const double* Ra_s, const
     return SDDC_OK;
   }
   const double* src;
-  if ((rc = prep_input(p, B, X_in, &src, s, p.Xa))) return rc;
-  if ((rc = launch_suffix(p, B, src, p.P, s))) return rc;
+  if ((rc = prep_state(p, B, X_in, p.Xa, p.P, &src, s))) return rc;
   for (int k = 0; k < nsteps; ++k) {
     if ((rc = step_once(p, B, Ra, Ra_s, src, X_out, linear, s))) return rc;
     src = X_out;
@@ -708,12 +692,13 @@ int sddc_diagnostics(sddc_plan* plan, int B, const double* X, double* out, void*
   int rc = check_batch(p, B);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  if ((rc = launch_suffix(p, B, X, p.Pa, s))) return rc;
+  if ((rc = launch_suffix(p, B, X, p.Pa, nullptr, s))) return rc;
   if ((rc = launch_spectral(p, B, X, p.Pa, nullptr, nullptr, 0, nullptr, p.slabs2, SDDC_FP64,
                             nullptr, nullptr, s)))
     return rc;
-  if ((rc = launch_ke_rows(p, B, p.slabs2, p.rowval, s))) return rc;
-  return launch_diag_final(p, B, X, p.rowval, out, s);
+  double* parts = p.L;   // 40 bytes per kDiagEntries entries
+  if ((rc = launch_ke_rows(p, B, X, p.slabs2, p.rowval, parts, s))) return rc;
+  return launch_diag_final(p, B, p.rowval, parts, out, s);
 }
 
 int sddc_run_stage(sddc_plan* plan, int B, int stage, const double* X, const double* Ra,
@@ -724,7 +709,7 @@ int sddc_run_stage(sddc_plan* plan, int B, int stage, const double* X, const dou
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   switch (stage) {
-    case 0: return launch_suffix(p, B, X, p.P, s);
+    case 0: return launch_suffix(p, B, X, p.P, nullptr, s);
     case 1:
       return launch_spectral(p, B, X, p.P, Ra, Ra_s, 1, p.L, p.slabs, p.precision, nullptr,
                              nullptr, s);

@@ -168,7 +168,8 @@ void free_tables(TableSet& t);
 FftShape make_shape(int L);
 
 // launchers implemented in the kernel translation units
-int launch_suffix(const Plan& p, int B, const double* X, double* P, hipStream_t s);
+// P of X; masked (may be null): of X under the symmetry mask, which goes there.
+int launch_suffix(const Plan& p, int B, const double* X, double* P, double* masked, hipStream_t s);
 int launch_spectral(const Plan& p, int B, const double* X, const double* P,
                     const double* Ra, const double* Ras, int want_linear, double* L,
                     void* slabs, int slab_precision, double* theta_out, double* slab9,
@@ -185,9 +186,13 @@ void free_chain(Plan& p);
 int launch_mask(const Plan& p, int B, const double* X, double* out, hipStream_t s);
 int launch_transform(const TableSet& t, int kind, int rows, int len_in, int n_out,
                      const double* in, double* out, hipStream_t s);
-int launch_ke_rows(const Plan& p, int B, const void* slabs64, double* rowval, hipStream_t s);
-int launch_diag_final(const Plan& p, int B, const double* X, const double* rowval,
-                      double* out, hipStream_t s);
+// Diagnostics: partial sums of a state, kDiagParts for each kDiagEntries entries
+constexpr int kDiagParts = 5, kDiagEntries = 2048;
+inline int diag_parts(const Plan& p) { return (3 * p.K * p.nr + kDiagEntries - 1) / kDiagEntries; }
+int launch_ke_rows(const Plan& p, int B, const double* X, const void* slabs64, double* rowval,
+                   double* parts, hipStream_t s);
+int launch_diag_final(const Plan& p, int B, const double* rowval, const double* parts, double* out,
+                      hipStream_t s);
 int nonlinear_lds_bytes(const Plan& p, int precision, int dfx);
 // sddc_step_linearized in two parts, for many dv about one X: the transforms'
 // input of X in the plan's workspace, then one dv.  Between the two no other call may

@@ -14,57 +14,90 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------------------
 // P[r] = sum_{m>r, m = r mod 2} psi[m]: the running sum f_e / b of A2_SINE,
 // A2_SINE_R2 and J_theta_RT (Matrix_Operators.py:222-231, 441-450, 502-511).
-// One workgroup per instance; threads (parity, i, segment): each segment is
-// summed, segment totals are scanned in LDS, then each segment is rewritten.
+// One workgroup per (row parity, 16 radial points, instance), threads (point,
+// segment of rows): a thread sums its rows, segment totals are scanned in LDS,
+// then the rows are rewritten.  With one workgroup per instance the lone CU's
+// loads took 13.5 us at N_fm = 512, N_r = 40 (5.7 here).  out (may be null): also the
+// masked state (Eq_SYM, Matrix_Operators.py:1054,1166); further workgroups copy
+// T and S.
 // ---------------------------------------------------------------------------
+constexpr int kSuffixCols = 16, kSuffixRows = 8, kSuffixCopy = 8;
+
 __global__ __launch_bounds__(1024) void k_suffix(const double* __restrict__ X,
-                                                 double* __restrict__ P, int K, int nr,
+                                                 double* __restrict__ P,
+                                                 double* __restrict__ out, int K, int nr,
                                                  int nseg) {
-  extern __shared__ double tot[];  // [nseg][2*nr]
-  const int b = blockIdx.x;
+  extern __shared__ double tot[];  // [nseg][kSuffixCols]
+  const int b = blockIdx.y, groups = (nr + kSuffixCols - 1) / kSuffixCols;
   const size_t N = (size_t)K * nr;
   const double* psi = X + (size_t)b * 3 * N;
-  double* Pb = P + (size_t)b * N;
-  const int lanes = 2 * nr;
-  const int t = threadIdx.x;
-  const int s = t / lanes;           // segment, 0 = highest rows
-  const int pi = t - s * lanes;
-  const int p = pi / nr, i = pi - p * nr;
-  const int top = ((K - 1) % 2 == p) ? K - 1 : K - 2;   // highest row of parity p
-  const int cnt = top / 2 + 1;                           // rows of parity p
-  const int per = (cnt + nseg - 1) / nseg;
-  const int r_hi = top - 2 * per * s;                    // first row of this segment
-  int nrows = 0;
-  if (s < nseg) {
-    nrows = cnt - per * s;
-    nrows = nrows < 0 ? 0 : (nrows > per ? per : nrows);
-    double acc = 0.0;
-    for (int q = 0; q < nrows; ++q) acc += psi[(size_t)(r_hi - 2 * q) * nr + i];
-    tot[s * lanes + pi] = acc;
+  if ((int)blockIdx.x >= 2 * groups) {   // T and S of a masked state: even rows stay
+    const size_t e0 = (size_t)(blockIdx.x - 2 * groups) * kSuffixCopy * blockDim.x + threadIdx.x;
+    double v[kSuffixCopy];
+#pragma unroll
+    for (int u = 0; u < kSuffixCopy; ++u) {
+      const size_t e = e0 + (size_t)u * blockDim.x;
+      v[u] = psi[N + (e < 2 * N ? e : 0)];
+    }
+#pragma unroll
+    for (int u = 0; u < kSuffixCopy; ++u) {
+      const size_t e = e0 + (size_t)u * blockDim.x;
+      const int k = (int)(e < N ? e : e - N) / nr;
+      if (e < 2 * N) out[(size_t)b * 3 * N + N + e] = k % 2 ? 0.0 : v[u];
+    }
+    return;
   }
-  __syncthreads();
-  if (s < nseg) {
-    double acc = 0.0;
-    for (int u = 0; u < s; ++u) acc += tot[u * lanes + pi];
-    for (int q = 0; q < nrows; ++q) {
-      const size_t o = (size_t)(r_hi - 2 * q) * nr + i;
-      Pb[o] = acc;
-      acc += psi[o];
+  const int p = blockIdx.x & 1, c = threadIdx.x % kSuffixCols, s = threadIdx.x / kSuffixCols;
+  const int i = (blockIdx.x >> 1) * kSuffixCols + c;   // segment 0: highest rows
+  const int top = ((K - 1) % 2 == p) ? K - 1 : K - 2;  // highest row of parity p
+  const int cnt = top / 2 + 1, per = (cnt + nseg - 1) / nseg;
+  const bool zero = out && p == 0;                     // psi keeps odd rows
+  int nrows = cnt - per * s;
+  nrows = nrows < 0 || i >= nr ? 0 : (nrows > per ? per : nrows);
+  const size_t o = (size_t)b * N + (i < nr ? i : 0);
+  const double* x = psi + (i < nr ? i : 0);
+  const int r0 = top - 2 * per * s;
+  double v[kSuffixRows], acc = 0.0;
+  auto load = [&](int q0) {
+#pragma unroll
+    for (int u = 0; u < kSuffixRows; ++u) {
+      const double w = x[(size_t)(q0 + u < nrows ? r0 - 2 * (q0 + u) : p) * nr];
+      v[u] = q0 + u < nrows && !zero ? w : 0.0;
+    }
+  };
+  for (int q0 = 0; q0 < per; q0 += kSuffixRows) {
+    load(q0);
+#pragma unroll
+    for (int u = 0; u < kSuffixRows; ++u) acc += v[u];
+  }
+  tot[s * kSuffixCols + c] = acc;
+  lds_barrier();
+  acc = 0.0;
+#pragma unroll 8
+  for (int u = 0; u < s; ++u) acc += tot[u * kSuffixCols + c];
+  for (int q0 = 0; q0 < per; q0 += kSuffixRows) {
+    if (per > kSuffixRows) load(q0);
+#pragma unroll
+    for (int u = 0; u < kSuffixRows; ++u) {
+      if (q0 + u >= nrows) break;
+      const size_t row = (size_t)(r0 - 2 * (q0 + u)) * nr;
+      P[o + row] = acc;
+      if (out) out[o + 2 * b * N + row] = v[u];
+      acc += v[u];
     }
   }
 }
 
-int launch_suffix(const Plan& p, int B, const double* X, double* P, hipStream_t s) {
+int launch_suffix(const Plan& p, int B, const double* X, double* P, double* masked,
+                  hipStream_t s) {
   if (B <= 0) return SDDC_OK;
-  const int lanes = 2 * p.nr;
-  int nseg = 1024 / lanes;
-  const int half = (p.K + 1) / 2;
-  const int want = (half + 7) / 8;   // at least 8 rows per segment
-  if (nseg > want) nseg = want;
-  if (nseg < 1) nseg = 1;
-  int threads = ((nseg * lanes + 63) / 64) * 64;
-  hipLaunchKernelGGL(k_suffix, dim3(B), dim3(threads), nseg * lanes * sizeof(double), s, X, P,
-                     p.K, p.nr, nseg);
+  const int half = (p.K + 1) / 2, want = (half + 3) / 4;   // four rows per segment
+  const int nseg = want > 64 ? 64 : (want < 4 ? 4 : want), threads = nseg * kSuffixCols;
+  const long long copy = masked ? 2LL * p.K * p.nr : 0, per = (long long)kSuffixCopy * threads;
+  const dim3 grid(2 * ((p.nr + kSuffixCols - 1) / kSuffixCols) + (unsigned)((copy + per - 1) / per),
+                  B);
+  hipLaunchKernelGGL(k_suffix, grid, dim3(threads), threads * sizeof(double), s, X, P, masked, p.K,
+                     p.nr, nseg);
   return hip_check(hipGetLastError(), "k_suffix");
 }
 
@@ -715,74 +748,53 @@ int launch_mask(const Plan& p, int B, const double* X, double* out, hipStream_t 
 // Diagnostics: ||X||_2, kinetic energy (radial trapezoid over the interior
 // points of the per-row theta integrals, Main.py:129-134) and Nu-1 of T and S
 // at R_1 and at R_2 (Main.py:52-68; the reference returns the R_1 value and
-// checks it against R_2).  One workgroup per instance; out[b] holds
-// (norm, KE, NuT(R_1), NuS(R_1), NuT(R_2), NuS(R_2)).
+// checks it against R_2), from the partial sums of k_ke_rows.  One wavefront per
+// instance; out[b] holds (norm, KE, NuT(R_1), NuS(R_1), NuT(R_2), NuS(R_2)).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_diag_final(const double* __restrict__ X,
-                                                    const double* __restrict__ rowval,
-                                                    const double* __restrict__ Dfull,
-                                                    const double* __restrict__ Rg, int K, int nr,
-                                                    double d, double* __restrict__ out) {
-  constexpr int NV = 6;
-  __shared__ double red[NV][256];
-  const int b = blockIdx.x;
-  const size_t N = (size_t)K * nr;
-  const double* Xb = X + (size_t)b * 3 * N;
-  const int Np1 = nr + 2;
-  const double* Dlast = Dfull + (size_t)(Np1 - 1) * Np1;   // row of R_2
-  double v[NV] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  for (size_t e = threadIdx.x; e < 3 * N; e += blockDim.x) v[0] += Xb[e] * Xb[e];
-  // Nusselt: sum over even k of (D[row,1:-1] . T_k) / (1 - k^2), rows 0 and N_r
-  for (int k = 2 * threadIdx.x; k < K; k += 2 * blockDim.x) {
-    double aT = 0.0, aS = 0.0, bT = 0.0, bS = 0.0;
-    for (int i = 0; i < nr; ++i) {
-      const double t = Xb[N + (size_t)k * nr + i], c = Xb[2 * N + (size_t)k * nr + i];
-      aT += Dfull[i + 1] * t;
-      aS += Dfull[i + 1] * c;
-      bT += Dlast[i + 1] * t;
-      bS += Dlast[i + 1] * c;
-    }
-    const double den = 1.0 - (double)k * (double)k;
-    v[2] += aT / den;
-    v[3] += aS / den;
-    v[4] += bT / den;
-    v[5] += bS / den;
-  }
-  for (int i = threadIdx.x; i < nr; i += blockDim.x) {
+__global__ __launch_bounds__(64) void k_diag_final(const double* __restrict__ rowval,
+                                                   const double* __restrict__ parts, int nparts,
+                                                   const double* __restrict__ Rg, int nr, double d,
+                                                   double* __restrict__ out) {
+  constexpr int NV = kDiagParts + 1;
+  const int b = blockIdx.x, Np1 = nr + 2;
+  double v[NV];
+#pragma unroll
+  for (int q = 0; q < NV; ++q) v[q] = 0.0;
+  for (int i = threadIdx.x; i < nr; i += 64) {
     const double* x = Rg + 1;   // interior points
     double w;
     if (nr == 1) w = 0.0;
     else if (i == 0) w = 0.5 * (x[1] - x[0]);
     else if (i == nr - 1) w = 0.5 * (x[nr - 1] - x[nr - 2]);
     else w = 0.5 * (x[i + 1] - x[i - 1]);
-    if (rowval) v[1] += w * rowval[(size_t)b * nr + i];
+    v[kDiagParts] += w * rowval[(size_t)b * nr + i];
   }
-  for (int q = 0; q < NV; ++q) red[q][threadIdx.x] = v[q];
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st)
-      for (int q = 0; q < NV; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + st];
-    __syncthreads();
-  }
+  for (int c = threadIdx.x; c < nparts; c += 64)
+#pragma unroll
+    for (int q = 0; q < kDiagParts; ++q) v[q] += parts[((size_t)b * nparts + c) * kDiagParts + q];
+#pragma unroll
+  for (int q = 0; q < NV; ++q)
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) v[q] += __shfl_xor(v[q], m);
   if (threadIdx.x == 0) {
     const double R1 = 1 / d, R2 = (1 + d) / d;
     const double A_T = (R1 * R2) / (R1 - R2);
     const double V = (2.0 / 3.0) * (Rg[Np1 - 1] * Rg[Np1 - 1] * Rg[Np1 - 1] - Rg[0] * Rg[0] * Rg[0]);
     const double c0 = (Rg[0] * Rg[0]) / A_T, c1 = (Rg[Np1 - 1] * Rg[Np1 - 1]) / A_T;
-    double* o = out + (size_t)b * NV;
-    o[0] = sqrt(red[0][0]);
-    o[1] = (0.5 / V) * red[1][0];
-    o[2] = c0 * red[2][0];
-    o[3] = c0 * red[3][0];
-    o[4] = c1 * red[4][0];
-    o[5] = c1 * red[5][0];
+    double* o = out + (size_t)b * 6;
+    o[0] = sqrt(v[0]);
+    o[1] = (0.5 / V) * v[kDiagParts];
+    o[2] = c0 * v[1];
+    o[3] = c0 * v[2];
+    o[4] = c1 * v[3];
+    o[5] = c1 * v[4];
   }
 }
 
-int launch_diag_final(const Plan& p, int B, const double* X, const double* rowval, double* out,
+int launch_diag_final(const Plan& p, int B, const double* rowval, const double* parts, double* out,
                       hipStream_t s) {
   if (B <= 0) return SDDC_OK;
-  hipLaunchKernelGGL(k_diag_final, dim3(B), dim3(256), 0, s, X, rowval, p.Dfull, p.R, p.K, p.nr,
+  hipLaunchKernelGGL(k_diag_final, dim3(B), dim3(64), 0, s, rowval, parts, diag_parts(p), p.R, p.nr,
                      p.d, out);
   return hip_check(hipGetLastError(), "k_diag_final");
 }

@@ -1391,13 +1391,56 @@ int launch_nonlinear(const Plan& p, int B, const void* slabs, const void* slabs2
 // Kinetic energy, one workgroup per (radial row i, instance b): synthesise
 // J_theta(psi)/r (cosine) and Dr psi (sine) on grid(3K), and integrate
 // (J^2 + D^2) sin(theta) over theta with the trapezoid rule
-// (Main.py:107-130).  The radial trapezoid is done in k_diag_final.
+// (Main.py:107-130).  The radial trapezoid is done in k_diag_final.  Workgroups
+// i >= nr form the state's own sums beside them, over kDiagEntries entries each
+// (one workgroup per instance, walking it mode by mode after this launch, took
+// 15 us at N_fm = 128, N_r = 30 and 53 us at 300, 48).
 // ---------------------------------------------------------------------------
+// parts[0..4] of the entries [e0, e0 + kDiagEntries) of a state: squares, and the
+// sums over even k of (D[row,1:-1] . T_k) / (1 - k^2) (S_k) for the rows of R_1 and R_2.
+__device__ __forceinline__ void diag_entries(const double* __restrict__ Xb,
+                                             const double* __restrict__ Dfull, int K, int nr,
+                                             int e0, double* red, double* __restrict__ parts) {
+  const int N = K * nr, Np1 = nr + 2;
+  const double* Dlast = Dfull + (size_t)(Np1 - 1) * Np1;   // row of R_2
+  constexpr int U = kDiagEntries / 256;
+  double x[U], v[kDiagParts] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int e = e0 + threadIdx.x + 256 * u;
+    x[u] = e < 3 * N ? Xb[e] : 0.0;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int e = e0 + threadIdx.x + 256 * u;
+    v[0] = fma(x[u], x[u], v[0]);
+    if (e < N || e >= 3 * N) continue;
+    const int f = e >= 2 * N, w = e - (1 + f) * N, k = w / nr, i = w - k * nr;
+    if (k % 2) continue;
+    const double t = x[u] / (1.0 - (double)k * (double)k);
+    v[1 + f] = fma(Dfull[i + 1], t, v[1 + f]);
+    v[3 + f] = fma(Dlast[i + 1], t, v[3 + f]);
+  }
+#pragma unroll
+  for (int q = 0; q < kDiagParts; ++q) {
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) v[q] += __shfl_xor(v[q], m);
+    if ((threadIdx.x & 63) == 0) red[4 * q + (threadIdx.x >> 6)] = v[q];
+  }
+  __syncthreads();
+  const int q = threadIdx.x;
+  if (q < kDiagParts)
+    parts[q] = (red[4 * q] + red[4 * q + 1]) + (red[4 * q + 2] + red[4 * q + 3]);
+}
+
 __global__ __launch_bounds__(256) void k_ke_rows(FftShape sh, const double2* tw_,
                                                  const double2* rot_, int K, int nr,
                                                  const double* __restrict__ slabs,
                                                  const double* __restrict__ vecs, int NRP,
-                                                 double* __restrict__ rowval) {
+                                                 double* __restrict__ rowval,
+                                                 const double* __restrict__ X,
+                                                 const double* __restrict__ Dfull,
+                                                 double* __restrict__ parts) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   using C = cplx<double>;
   __shared__ double red[256];
@@ -1408,6 +1451,12 @@ __global__ __launch_bounds__(256) void k_ke_rows(FftShape sh, const double2* tw_
   const C* tw = reinterpret_cast<const C*>(tw_);
   const C* rot = reinterpret_cast<const C*>(rot_);
   const int i = blockIdx.x, b = blockIdx.y;
+  if (i >= nr) {
+    const int c = i - nr, nc = gridDim.x - nr;
+    diag_entries(X + (size_t)b * 3 * K * nr, Dfull, K, nr, c * kDiagEntries, red,
+                 parts + ((size_t)b * nc + c) * kDiagParts);
+    return;
+  }
   const double* jt = slabs + ((size_t)(b * 7 + 0) * nr + i) * K;
   const double* dp = slabs + ((size_t)(b * 7 + 1) * nr + i) * K;
   // IR@JPSI = (1/R_i) * JPSI (Main.py:102,112)
@@ -1450,13 +1499,15 @@ __global__ __launch_bounds__(256) void k_ke_rows(FftShape sh, const double2* tw_
   if (threadIdx.x == 0) rowval[(size_t)b * nr + i] = red[0];
 }
 
-int launch_ke_rows(const Plan& p, int B, const void* slabs64, double* rowval, hipStream_t s) {
+int launch_ke_rows(const Plan& p, int B, const double* X, const void* slabs64, double* rowval,
+                   double* parts, hipStream_t s) {
   const size_t lds = 2 * (size_t)p.tabKE.L * sizeof(double2);
   if (lds > 160 * 1024) return fail(SDDC_ERR_UNSUPPORTED, "N_fm too large for the LDS energy kernel");
   static std::atomic<size_t> cur{0};
   if (int rc = ensure_dynamic_lds((const void*)k_ke_rows, lds, cur)) return rc;
-  hipLaunchKernelGGL(k_ke_rows, dim3(p.nr, B), dim3(256), lds, s, p.tabKE.shape, p.tabKE.tw64,
-                     p.tabKE.rot64, p.K, p.nr, (const double*)slabs64, p.vecs, p.NRP, rowval);
+  hipLaunchKernelGGL(k_ke_rows, dim3(p.nr + diag_parts(p), B), dim3(256), lds, s, p.tabKE.shape,
+                     p.tabKE.tw64, p.tabKE.rot64, p.K, p.nr, (const double*)slabs64, p.vecs, p.NRP,
+                     rowval, X, p.Dfull, parts);
   return hip_check(hipGetLastError(), "k_ke_rows");
 }
 
