@@ -333,6 +333,10 @@ int sddc_run_stage(sddc_plan* plan, int B, int stage, const double* X, const dou
 const char* sddc_last_error(void);
 const char* sddc_version(void);
 
+/* Bob Jenkins' lookup3 hashlittle (the published hash) of n bytes: the checksum
+ * of HDF5's metadata, for the checkpoint writer.  Host memory. */
+int sddc_lookup3(const char* data, long long n, unsigned initval, unsigned* hash);
+
 #ifdef __cplusplus
 }
 #endif

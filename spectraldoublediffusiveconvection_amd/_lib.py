@@ -121,6 +121,8 @@ _SIGS = {
                                  ctypes.POINTER(SddcArclengthInfo), _V]),
     "sddc_last_error": (ctypes.c_char_p, []),
     "sddc_version": (ctypes.c_char_p, []),
+    "sddc_lookup3": (_I, [ctypes.c_char_p, ctypes.c_longlong, ctypes.c_uint,
+                          ctypes.POINTER(ctypes.c_uint)]),
 }
 
 EXPORTED = tuple(_SIGS)

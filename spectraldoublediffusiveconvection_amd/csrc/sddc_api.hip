@@ -207,6 +207,37 @@ static int static_scratch(int dev, unsigned char** out);
 const char* sddc_last_error(void) { return g_last_error.c_str(); }
 const char* sddc_version(void) { return "sddc 0.1 gfx950"; }
 
+int sddc_lookup3(const char* data, long long n, unsigned initval, unsigned* hash) {
+  if (!hash || n < 0 || (n > 0 && !data)) return fail(SDDC_ERR_INVALID, "bad argument");
+  auto rot = [](unsigned x, int k) { return (x << k) | (x >> (32 - k)); };
+  unsigned s[3];
+  s[0] = s[1] = s[2] = 0xDEADBEEFu + (unsigned)n + initval;
+  unsigned &a = s[0], &b = s[1], &c = s[2];
+  *hash = c;
+  if (n == 0) return SDDC_OK;
+  // blocks of three little-endian words; the last one is padded with zeros
+  for (long long i = 0; i < n; i += 12) {
+    for (long long q = i; q < n && q < i + 12; ++q)
+      s[(q - i) / 4] += (unsigned)(unsigned char)data[q] << 8 * ((q - i) % 4);
+    if (i + 12 >= n) break;
+    const int mix[6] = {4, 6, 8, 16, 19, 4};
+    for (int m = 0; m < 6; ++m) {   // (a, c, b), (b, a, c), (c, b, a) in turn
+      unsigned &x = s[m % 3], &y = s[(m + 2) % 3], &z = s[(m + 1) % 3];
+      x -= y;
+      x ^= rot(y, mix[m]);
+      y += z;
+    }
+  }
+  const int fin[7] = {14, 11, 25, 16, 4, 14, 24};
+  for (int m = 0; m < 7; ++m) {     // (c, b), (a, c), (b, a) in turn
+    unsigned &x = s[(m + 2) % 3], &y = s[(m + 1) % 3];
+    x ^= y;
+    x -= rot(y, fin[m]);
+  }
+  *hash = c;
+  return SDDC_OK;
+}
+
 int sddc_plan_create(const sddc_operators* ops, int precision, int symmetric, int max_batch,
                      sddc_plan** out) {
   return sddc_plan_create_tuned(ops, precision, symmetric, max_batch, nullptr, out);

@@ -16,10 +16,13 @@ the same groups and datasets, readable by h5py).
 """
 from __future__ import annotations
 
-import time
-
 import numpy as np
 import torch
+
+try:
+    import h5py
+except ImportError:   # the package's own writer then
+    h5py = None
 
 from .. import operators as _ops
 from . import Matrix_Operators as _mo
@@ -97,11 +100,10 @@ def Build_Matrix_Operators(N_fm, N_r, d, dt, Pr, Tau):
             list(ops.Linv_S), args_A4, args_FXS)
 
 
+_FETCH = 64   # steps whose diagnostics may be queued
+
+
 def _write_checkpoint(save_filename, X_DATA, scalars, params):
-    try:
-        import h5py
-    except ImportError:
-        h5py = None
     if h5py is not None:
         with h5py.File(save_filename, "w") as f:
             f.create_group("Checkpoints")["X_DATA"] = X_DATA
@@ -128,33 +130,50 @@ def _Time_Step(X, Ra, Ra_s, Tau, Pr, d, N_fm, N_r, symmetric, save_filename='Tim
     N_print = 10
     x = _dev(X)
     xn = torch.empty_like(x)
+    ra, ras = plan._params(Ra, 1), plan._params(Ra_s, 1)
     Time, X_DATA, KE, NuT, NuS, Norm = [], [], [], [], [], []
     params = {"Ra": Ra, "Ra_s": Ra_s, "Tau": Tau, "Pr": Pr, "d": d, "N_r": N_r, "N_fm": N_fm,
               "dt": dt, "start_time": start_time, "symmetric": symmetric}
-    timer = 0.0
+    # Steps and diagnostics are queued; their values and times are fetched where
+    # they are used (prints, checkpoints, the end) and every _FETCH steps.
+    timer, queued = 0.0, []
+    marks = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
+             for _ in range(min(N_iters, _FETCH))]
+
+    def fetch():
+        if not queued:
+            return 0.0
+        for dg in torch.cat(queued).cpu().numpy():   # waits for the queue
+            Norm.append(dg[0])
+            KE.append(dg[1])
+            NuT.append(dg[2])
+            NuS.append(dg[3])
+        first = 1 if len(Norm) == len(queued) else 0   # the first step is not timed
+        spent = sum(st.elapsed_time(end) for st, end in marks[first:len(queued)])
+        queued.clear()
+        return 1e-3 * spent
+
     X_new = np.asarray(X, dtype=np.float64)
     for iteration in range(N_iters):
-        torch.cuda.synchronize()
-        st = time.time()
-        plan.step(x, Ra, Ra_s, nsteps=1, linear=linear, out=xn)
-        torch.cuda.synchronize()
-        end = time.time()
-        dg = _host(plan.diagnostics(xn))
-        Norm.append(dg[0])
-        KE.append(dg[1])
-        NuT.append(dg[2])
-        NuS.append(dg[3])
+        st, end = marks[len(queued)]
+        st.record()
+        plan.step(x, ra, ras, nsteps=1, linear=linear, out=xn)
+        end.record()
+        queued.append(plan.diagnostics(xn))
         Time.append(start_time + dt * iteration)
-        if (iteration % N_print == 0) and (Verbose is True):
+        printing = (iteration % N_print == 0) and (Verbose is True)
+        saving = iteration % N_save == 0
+        if printing or saving or len(queued) == _FETCH:
+            timer += fetch()
+        if printing:
             print("Iteration =%i, Time = %e, Energy = %e, NuT = %e \n " %
                   (iteration, start_time + dt * iteration, KE[-1], NuT[-1]))
-        if iteration % N_save == 0:
+        if saving:
             X_DATA.append(_host(xn))
             _write_checkpoint(save_filename, X_DATA, {"Norm": Norm, "KE": KE, "Nu_T": NuT,
                                                       "Nu_S": NuS, "Time": Time}, params)
         x, xn = xn, x   # the step already applied the symmetry mask
-        if iteration > 0:
-            timer += end - st
+    timer += fetch()
     if N_iters > 1:
         print("Avg time = %e \n" % (timer / (N_iters - 1)))
     if N_iters > 0:
@@ -329,10 +348,6 @@ def _ContinC(Y_0_dot, Y_0, sign, ds, Ra, Ra_s, Tau, Pr, d, N_fm, N_r, symmetric,
 
 def _write_continuation(filename, Result, params):
     """Checkpoints, Parameters and Bifurcation groups (Main.py:1024-1040)."""
-    try:
-        import h5py
-    except ImportError:
-        h5py = None
     if h5py is not None:
         with h5py.File(filename, "w") as f:
             g = f.create_group("Checkpoints")

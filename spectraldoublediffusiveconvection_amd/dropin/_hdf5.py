@@ -22,51 +22,24 @@ sequences to arrays of those.  Strings become fixed-length UTF-8 strings
 (h5py would write variable-length ones, which need a global heap; h5py reads
 these back as bytes).
 """
+import ctypes
 import struct
 
 import numpy as np
 
+from .. import _lib
+
 UNDEF = 0xFFFFFFFFFFFFFFFF
-_M = 0xFFFFFFFF
-
-
-def _rot(x, k):
-    return ((x << k) | (x >> (32 - k))) & _M
 
 
 def lookup3(data, initval=0):
     """Bob Jenkins' lookup3 hashlittle over bytes, as HDF5 checksums its
-    metadata (byte-wise form: the value does not depend on alignment)."""
+    metadata (sddc_lookup3: in Python the 21 headers of a checkpoint took
+    0.8 ms)."""
     k = bytes(data)
-    n = len(k)
-    a = b = c = (0xDEADBEEF + n + initval) & _M
-    i = 0
-    while n > 12:
-        a = (a + int.from_bytes(k[i:i + 4], "little")) & _M
-        b = (b + int.from_bytes(k[i + 4:i + 8], "little")) & _M
-        c = (c + int.from_bytes(k[i + 8:i + 12], "little")) & _M
-        a = (a - c) & _M; a ^= _rot(c, 4); c = (c + b) & _M
-        b = (b - a) & _M; b ^= _rot(a, 6); a = (a + c) & _M
-        c = (c - b) & _M; c ^= _rot(b, 8); b = (b + a) & _M
-        a = (a - c) & _M; a ^= _rot(c, 16); c = (c + b) & _M
-        b = (b - a) & _M; b ^= _rot(a, 19); a = (a + c) & _M
-        c = (c - b) & _M; c ^= _rot(b, 4); b = (b + a) & _M
-        n -= 12
-        i += 12
-    if n == 0:
-        return c
-    tail = k[i:i + n] + bytes(12 - n)
-    a = (a + int.from_bytes(tail[0:4], "little")) & _M
-    b = (b + int.from_bytes(tail[4:8], "little")) & _M
-    c = (c + int.from_bytes(tail[8:12], "little")) & _M
-    c ^= b; c = (c - _rot(b, 14)) & _M
-    a ^= c; a = (a - _rot(c, 11)) & _M
-    b ^= a; b = (b - _rot(a, 25)) & _M
-    c ^= b; c = (c - _rot(b, 16)) & _M
-    a ^= c; a = (a - _rot(c, 4)) & _M
-    b ^= a; b = (b - _rot(a, 14)) & _M
-    c ^= b; c = (c - _rot(b, 24)) & _M
-    return c
+    h = ctypes.c_uint()
+    _lib.check(_lib.lib().sddc_lookup3(k, len(k), initval, ctypes.byref(h)))
+    return h.value
 
 
 # ---------------------------------------------------------------------------
@@ -126,7 +99,8 @@ def _layout(addr, size):
 
 
 def _encode(value):
-    """(datatype message body, shape, raw little-endian bytes) of a value."""
+    """(datatype message body, shape, raw little-endian bytes or a view of them)
+    of a value."""
     if isinstance(value, (str, bytes)):
         raw = value.encode("utf-8") if isinstance(value, str) else bytes(value)
         size = max(len(raw), 1)
@@ -139,7 +113,8 @@ def _encode(value):
     if np.issubdtype(arr.dtype, np.integer):
         return _int_type(8), arr.shape, arr.astype("<i8").tobytes()
     if np.issubdtype(arr.dtype, np.floating):
-        return _float64_type(), arr.shape, arr.astype("<f8").tobytes()
+        raw = np.ascontiguousarray(arr, dtype="<f8")
+        return _float64_type(), arr.shape, memoryview(raw).cast("B") if raw.size else b""
     raise TypeError("unsupported value type %s" % arr.dtype)
 
 
