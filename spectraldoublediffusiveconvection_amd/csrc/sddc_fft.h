@@ -312,6 +312,15 @@ __device__ __forceinline__ void wave_lds_sync() {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
+// The same among the G wavefronts of a transform (G > 1: the workgroup).
+template <int G>
+__device__ __forceinline__ void group_lds_sync() {
+  if (G == 1)
+    wave_lds_sync();
+  else
+    lds_barrier();
+}
+
 // Iterations are processed in chunks of U: every LDS read of a chunk (data
 // and twiddles, indices clamped in range) is issued before any is used, so
 // one wavefront keeps several reads in flight; only stores are predicated.
@@ -486,21 +495,22 @@ __device__ void fft_run_ip(cplx<R>* buf, const FftShape& sh, const cplx<R>* __re
 }
 
 // ---------------------------------------------------------------------------
-// The in-place transform of any length up to 64 NC with factors 2, 3, 4 and 5:
-// chunk counts fixed by NC, the schedule make_shape's, the twiddles in the
-// per-pass layout (ip_twiddle_offset) in LDS.
+// The in-place transform of any length up to 64 G NC with factors 2, 3, 4 and 5 by
+// one wavefront or a workgroup of G: chunk counts fixed by NC, the schedule
+// make_shape's, the twiddles in the per-pass layout (ip_twiddle_offset) in LDS.
+// lane: the thread's place among the 64 G.
 // ---------------------------------------------------------------------------
-template <typename R, int NC, int RADIX>
+template <typename R, int NC, int RADIX, int G>
 __device__ __forceinline__ void fft_pass_nc(cplx<R>* buf, int L, int Ns,
                                             const cplx<R>* __restrict__ tw, bool inv, int lane) {
-  constexpr int U = (NC + RADIX - 1) / RADIX;   // chunks of 64 butterflies
+  constexpr int U = (NC + RADIX - 1) / RADIX;   // chunks of 64 G butterflies
   const int nb = L / RADIX;
   const float rns = 1.0f / (float)Ns;
   cplx<R> v[U][RADIX], w[U][RADIX];
   int base[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int jr = lane + 64 * u;
+    const int jr = lane + 64 * G * u;
     const int j = jr < nb ? jr : nb - 1;
     const int jq = qdiv(j, Ns, rns);
     const int k = j - jq * Ns;
@@ -510,6 +520,7 @@ __device__ __forceinline__ void fft_pass_nc(cplx<R>* buf, int L, int Ns,
 #pragma unroll
     for (int s = 1; s < RADIX; ++s) w[u][s] = tw_get(tw, (s - 1) * Ns + k, inv);
   }
+  if (G > 1) lds_barrier();   // every read before the first write
 #pragma unroll
   for (int u = 0; u < U; ++u) {
 #pragma unroll
@@ -521,26 +532,26 @@ __device__ __forceinline__ void fft_pass_nc(cplx<R>* buf, int L, int Ns,
   }
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    if (lane + 64 * u < nb)
+    if (lane + 64 * G * u < nb)
 #pragma unroll
       for (int s = 0; s < RADIX; ++s) buf[base[u] + s * Ns] = v[u][s];
 }
 
-template <typename R, int NC>
+template <typename R, int NC, int G = 1>
 __device__ __forceinline__ void fft_run_nc(cplx<R>* buf, const FftShape& sh,
                                            const cplx<R>* __restrict__ tw, bool inv, int lane) {
   int Ns = 1;
   for (int p = 0; p < sh.npass; ++p) {
     const int r = sh.radix[p];
     if (r == 4)
-      fft_pass_nc<R, NC, 4>(buf, sh.L, Ns, tw, inv, lane);
+      fft_pass_nc<R, NC, 4, G>(buf, sh.L, Ns, tw, inv, lane);
     else if (r == 2)
-      fft_pass_nc<R, NC, 2>(buf, sh.L, Ns, tw, inv, lane);
+      fft_pass_nc<R, NC, 2, G>(buf, sh.L, Ns, tw, inv, lane);
     else if (r == 3)
-      fft_pass_nc<R, NC, 3>(buf, sh.L, Ns, tw, inv, lane);
+      fft_pass_nc<R, NC, 3, G>(buf, sh.L, Ns, tw, inv, lane);
     else
-      fft_pass_nc<R, NC, 5>(buf, sh.L, Ns, tw, inv, lane);
-    wave_lds_sync();
+      fft_pass_nc<R, NC, 5, G>(buf, sh.L, Ns, tw, inv, lane);
+    group_lds_sync<G>();
     tw += (r - 1) * Ns;
     Ns *= r;
   }
@@ -583,18 +594,18 @@ __host__ __device__ constexpr int ip_twiddle_offset(int L, int P) {
   return off;
 }
 
-template <typename R, int L, int RADIX, int NS, int TWO>
+template <typename R, int L, int RADIX, int NS, int TWO, int G>
 __device__ __forceinline__ void fft_pass_ct(cplx<R>* buf, const cplx<R>* __restrict__ tw,
                                             bool inv, int lane) {
   constexpr int NB = L / RADIX;                 // butterflies
-  constexpr int U = (NB + 63) / 64;             // chunks of 64 butterflies
+  constexpr int W = 64 * G, U = (NB + W - 1) / W;   // chunks of W butterflies
   static_assert(U <= IpChunk<RADIX>::U, "in-place chunk exceeds the register budget");
   cplx<R> v[U][RADIX], w[U][RADIX];
   int base[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int jr = lane + 64 * u;
-    const int j = (NB % 64 == 0 || jr < NB) ? jr : NB - 1;
+    const int jr = lane + W * u;
+    const int j = (NB % W == 0 || jr < NB) ? jr : NB - 1;
     const int jq = j / NS;
     const int k = j - jq * NS;
     base[u] = jq * NS * RADIX + k;
@@ -605,6 +616,7 @@ __device__ __forceinline__ void fft_pass_ct(cplx<R>* buf, const cplx<R>* __restr
 #pragma unroll
       for (int s = 1; s < RADIX; ++s) w[u][s] = tw_get(tw, TWO + (s - 1) * NS + k, inv);
   }
+  if (G > 1) lds_barrier();   // every read before the first write
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if constexpr (NS > 1)
@@ -617,20 +629,20 @@ __device__ __forceinline__ void fft_pass_ct(cplx<R>* buf, const cplx<R>* __restr
   }
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    if (NB % 64 == 0 || lane + 64 * u < NB)
+    if (NB % W == 0 || lane + W * u < NB)
 #pragma unroll
       for (int s = 0; s < RADIX; ++s) buf[base[u] + s * NS] = v[u][s];
 }
 
 // All passes; tw is the per-pass twiddle table (ip_twiddle_offset).
-template <typename R, int L, int P = 0, int NS = 1>
+template <typename R, int L, int P = 0, int NS = 1, int G = 1>
 __device__ __forceinline__ void fft_run_ct(cplx<R>* buf, const cplx<R>* __restrict__ tw, bool inv,
                                            int lane) {
   if constexpr (P < ip_npass(L)) {
     constexpr int RADIX = ip_radix(L, P);
-    fft_pass_ct<R, L, RADIX, NS, ip_twiddle_offset(L, P)>(buf, tw, inv, lane);
-    wave_lds_sync();
-    fft_run_ct<R, L, P + 1, NS * RADIX>(buf, tw, inv, lane);
+    fft_pass_ct<R, L, RADIX, NS, ip_twiddle_offset(L, P), G>(buf, tw, inv, lane);
+    group_lds_sync<G>();
+    fft_run_ct<R, L, P + 1, NS * RADIX, G>(buf, tw, inv, lane);
   }
 }
 

@@ -87,9 +87,221 @@ __global__ __launch_bounds__(256) void k_transform(FftShape sh, const double2* t
   }
 }
 
+// The same for lengths up to 64 G NC with factors 2, 3 and 5, in place, G
+// wavefronts per two rows; LCT: the length, when it is one whose passes are
+// compiled (0: any).  Grid values pass through LDS in the reordered layout and
+// memory in order.  The passes are bound by instruction issue (a variant that
+// kept their writes off shared LDS banks was slower), so the choice is how many
+// wavefronts share them, see launch_transform.
+constexpr int kTransformWaves = 4;
+
+template <int NC, int G, int LCT>
+__global__ __launch_bounds__(64 * kTransformWaves) void k_transform_nc(
+    FftShape sh, const double2* tw_, const double2* rot_, int kind, int rows, int len_in, int n_out,
+    const double* __restrict__ in, double* __restrict__ out) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  using C = cplx<double>;
+  constexpr int NTHR = 64 * kTransformWaves, NT = (64 * G * NC + NTHR - 1) / NTHR, W = 64 * G;
+  constexpr int PER = kTransformWaves / G;   // transforms of a workgroup
+  __shared__ int ex[2][kTransformWaves];
+  const int L = LCT ? LCT : sh.L, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), grp = wave / G;
+  const int lane = threadIdx.x % W;
+  C* tw = reinterpret_cast<C*>(smem_raw);
+  C* A = tw + (size_t)(1 + grp) * L;
+  const C* rot = reinterpret_cast<const C*>(rot_);
+  C twr[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int k = threadIdx.x + NTHR * j;
+    twr[j] = reinterpret_cast<const C*>(tw_)[k < L ? k : L - 1];
+  }
+  const int r0 = 2 * (blockIdx.x * PER + grp), rc = r0 < rows ? r0 : rows - 1;
+  const bool two = r0 + 1 < rows;
+  const double* u = in + (size_t)rc * len_in;
+  const double* v = two ? u + len_in : u;
+  const bool synthesis = kind == SDDC_IDCT || kind == SDDC_IDST;
+  const bool is_sin = kind == SDDC_IDST || kind == SDDC_DST;
+  // IDCT with n < len_in keeps the first n coefficients (DCT-III truncation)
+  const int K = len_in < L ? len_in : L;
+  double du[NC], dv[NC];
+  C rr[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int k = lane + W * c, kc = k < K ? k : K - 1;
+    du[c] = u[kc];
+    dv[c] = v[kc];
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) rr[c] = rot[lane + W * c < L ? lane + W * c : L - 1];
+  int eu = -1000, ev = -1000;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int k = lane + W * c;
+    if (k >= K || (synthesis && is_sin && k == 0)) du[c] = dv[c] = 0.0;
+    if (!two) dv[c] = 0.0;
+    eu = max(eu, bexp(du[c]));
+    ev = max(ev, bexp(dv[c]));
+  }
+  eu = __ockl_wfred_max_i32(eu);
+  ev = __ockl_wfred_max_i32(ev);
+  if (G > 1) {
+    if ((threadIdx.x & 63) == 0) {
+      ex[0][wave] = eu;
+      ex[1][wave] = ev;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int w = 0; w < G; ++w) {
+      eu = max(eu, ex[0][w]);
+      ev = max(ev, ex[1][w]);
+    }
+  }
+  const double su = pow2_scale_e<double>(eu), sv = pow2_scale_e<double>(ev);
+  const double iu = 1.0 / su, iv = 1.0 / sv;
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    if (threadIdx.x + NTHR * j < L) tw[threadIdx.x + NTHR * j] = twr[j];
+  if (synthesis) {
+    double* cu = reinterpret_cast<double*>(A);   // K pairs of reals
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int k = lane + W * c;
+      du[c] = su * (k == 0 ? du[c] : 0.5 * du[c]);
+      dv[c] = sv * (k == 0 ? dv[c] : 0.5 * dv[c]);
+      if (k < K) {
+        cu[k] = du[c];
+        cu[K + k] = dv[c];
+      }
+    }
+    group_lds_sync<G>();
+    double mu[NC], mv[NC];   // mirrored: index L - k
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int m = L - (lane + W * c);
+      const bool ok = m > 0 && m < K;
+      mu[c] = cu[ok ? m : 0];
+      mv[c] = cu[K + (ok ? m : 0)];
+      if (!ok) mu[c] = mv[c] = 0.0;
+    }
+    group_lds_sync<G>();
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int k = lane + W * c;
+      const double au = is_sin ? mu[c] : du[c], av = is_sin ? mv[c] : dv[c];
+      const double aum = k ? (is_sin ? du[c] : mu[c]) : 0.0;
+      const double avm = k ? (is_sin ? dv[c] : mv[c]) : 0.0;
+      if (k < L) A[k] = cmul(C{au + avm, av - aum}, rr[c]);
+    }
+    __syncthreads();   // twiddles in LDS
+    if constexpr (LCT)
+      fft_run_ct<double, LCT, 0, 1, G>(A, tw, true, lane);
+    else
+      fft_run_nc<double, NC, G>(A, sh, tw, true, lane);
+    if (r0 >= rows) return;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int n = lane + W * c;
+      if (n >= L) break;
+      const C w = A[n % 2 ? L - 1 - n / 2 : n / 2];
+      const double sg = is_sin && n % 2 ? -1.0 : 1.0;
+      out[(size_t)r0 * n_out + n] = w.x * iu * sg;
+      if (two) out[(size_t)(r0 + 1) * n_out + n] = w.y * iv * sg;
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int n = lane + W * c;
+      const double sg = is_sin && n % 2 ? -1.0 : 1.0;
+      if (n < L) A[n % 2 ? L - 1 - n / 2 : n / 2] = {su * du[c] * sg, sv * dv[c] * sg};
+    }
+    __syncthreads();   // twiddles in LDS
+    if constexpr (LCT)
+      fft_run_ct<double, LCT, 0, 1, G>(A, tw, false, lane);
+    else
+      fft_run_nc<double, NC, G>(A, sh, tw, false, lane);
+    if (r0 >= rows) return;
+    const int nk = n_out < L ? n_out : L;
+    const double invL = 1.0 / L;
+    if (is_sin) {   // read at index L - k
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int k = lane + W * c < L ? lane + W * c : L - 1;
+        rr[c] = rot[k ? L - k : 0];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int k = lane + W * c;
+      if (k >= nk) break;
+      const int ka = is_sin && k ? L - k : k;
+      const C za = A[ka], zb = A[ka ? L - ka : 0];
+      // X = (a + conj b)/2, Y = (a - conj b)/(2i); C = Re(conj(e) X), Re(conj(e) Y)
+      const double c1 = rr[c].x * (0.5 * (za.x + zb.x)) + rr[c].y * (0.5 * (za.y - zb.y));
+      const double c2 = rr[c].x * (0.5 * (za.y + zb.y)) + rr[c].y * (-0.5 * (za.x - zb.x));
+      double a1 = (2.0 * (c1 * iu)) * invL, a2 = (2.0 * (c2 * iv)) * invL;
+      if (k == 0) {
+        a1 = is_sin ? 0.0 : 0.5 * a1;
+        a2 = is_sin ? 0.0 : 0.5 * a2;
+      }
+      out[(size_t)r0 * nk + k] = a1;
+      if (two) out[(size_t)(r0 + 1) * nk + k] = a2;
+    }
+  }
+}
+
+template <int NC, int G, int LCT = 0>
+static int launch_transform_nc(const TableSet& t, int kind, int rows, int len_in, int n_out,
+                               const double* in, double* out, hipStream_t s) {
+  const size_t lds = (1 + kTransformWaves / G) * (size_t)t.L * sizeof(double2);
+  static std::atomic<size_t> cur{0};
+  if (int rc = ensure_dynamic_lds((const void*)k_transform_nc<NC, G, LCT>, lds, cur)) return rc;
+  const int per = 2 * (kTransformWaves / G);
+  hipLaunchKernelGGL((k_transform_nc<NC, G, LCT>), dim3((rows + per - 1) / per), dim3(64 * kTransformWaves),
+                     lds, s, t.shape, t.twp64, t.rot64, kind, rows, len_in, n_out, in, out);
+  return hip_check(hipGetLastError(), "k_transform_nc");
+}
+
+// 0 when the length is not one of k_transform_nc's.
+static int transform_columns(const TableSet& t) {
+  for (int q = 0; q < t.shape.npass; ++q)
+    if (t.shape.radix[q] > 5) return 0;
+  const int nc = (t.L + 63) / 64;
+  return t.shape.npass > 0 && nc <= 32 ? nc : 0;
+}
+
 int launch_transform(const TableSet& t, int kind, int rows, int len_in, int n_out,
                      const double* in, double* out, hipStream_t s) {
   if (rows <= 0) return SDDC_OK;
+  if (const int nc = transform_columns(t)) {
+    auto run = [&](auto launch) { return launch(t, kind, rows, len_in, n_out, in, out, s); };
+    // Few rows leave SIMDs idle: four wavefronts share a transform.  Many rows: one,
+    // without workgroup barriers, while its registers leave room for others (8
+    // columns); longer ones keep k_transform.  One transform, us, before and now:
+    //   length   24   96  192  384  450  768  810
+    //   1 row   4.7  5.2  5.5  6.4  6.6  7.4  9.2   4.6  4.4  4.2  4.4  5.4  4.7  7.3
+    //   2496    6.5  7.3  7.9 11.1 12.2 16.1 19.7   4.5  5.1  5.1  8.6 11.9 13.5 19.7
+    //   10000    18   22   24   35   40   52   62   5.7  8.6  9.3   18   28   32   62
+    const bool few = rows <= 2048;
+    if (t.L == 192) return run(launch_transform_nc<3, 1, 192>);
+    if (t.L == 384)
+      return few ? run(launch_transform_nc<2, 4, 384>) : run(launch_transform_nc<6, 1, 384>);
+    if (t.L == 768)
+      return rows <= 4096 ? run(launch_transform_nc<3, 4, 768>)
+                          : run(launch_transform_nc<12, 1, 768>);
+    if (nc <= 1) return run(launch_transform_nc<1, 1>);
+    if (nc <= 2) return run(launch_transform_nc<2, 1>);
+    if (nc <= 3) return run(launch_transform_nc<3, 1>);
+    if (few) {
+      if (nc <= 4) return run(launch_transform_nc<1, 4>);
+      if (nc <= 8) return run(launch_transform_nc<2, 4>);
+      if (nc <= 12) return run(launch_transform_nc<3, 4>);
+      if (nc <= 16) return run(launch_transform_nc<4, 4>);
+      if (nc <= 24) return run(launch_transform_nc<6, 4>);
+      return run(launch_transform_nc<8, 4>);
+    }
+    if (nc <= 6) return run(launch_transform_nc<6, 1>);
+    if (nc <= 8) return run(launch_transform_nc<8, 1>);
+  }
   const size_t lds = 2 * (size_t)t.L * sizeof(double2);
   if (lds > 160 * 1024) return fail(SDDC_ERR_UNSUPPORTED, "transform length too large for LDS");
   static std::atomic<size_t> cur{0};
@@ -1217,10 +1429,15 @@ __global__ __launch_bounds__(DFX ? 640 : 320) void k_nonlinear_nc(
   nc_forward_project<R, NC>(o, buf + (size_t)(3 + q) * L, q, tw, sh, rot_g, F, b, i, nr, K, lane);
 }
 
+template <typename R, bool DFX>
+static size_t nl_nc_lds(int L) {
+  return (DFX ? 11 : 6) * (size_t)L * sizeof(cplx<R>);
+}
+
 template <typename R, int NC, bool DFX>
 static int launch_nl_nc(const Plan& p, int B, const void* slabs, const void* slabs2, void* F,
                         hipStream_t s, const cplx<R>* tw, const cplx<R>* rot) {
-  const size_t lds = (DFX ? 11 : 6) * (size_t)p.M * sizeof(cplx<R>);
+  const size_t lds = nl_nc_lds<R, DFX>(p.M);
   static std::atomic<size_t> cur{0};
   if (int rc = ensure_dynamic_lds((const void*)k_nonlinear_nc<R, NC, DFX>, lds, cur)) return rc;
   hipLaunchKernelGGL((k_nonlinear_nc<R, NC, DFX>), dim3(p.nr, B), dim3(DFX ? 640 : 320), lds, s,
@@ -1241,7 +1458,7 @@ static bool nl_nc_fits(const Plan& p) {
   for (int q = 0; q < sh.npass; ++q)
     if (sh.radix[q] > 5) return false;
   return sh.npass > 0 && 3 * p.K == 2 * sh.L && sh.L <= (F64 ? 64 * 13 : DFX ? 0 : 64 * 8) &&
-         (DFX ? 11 : 6) * (size_t)p.M * sizeof(cplx<R>) + 512 <= 160 * 1024;
+         nl_nc_lds<R, DFX>(p.M) + 512 <= 160 * 1024;
 }
 
 template <typename R, bool DFX>
