@@ -103,7 +103,8 @@ typedef struct sddc_plan sddc_plan;
  *                    sixteen per NAB2 workgroup.  The same bits whatever
  *                    the value
  *   sub_batches      graphs only: the batch is split into this many parts
- *                    (1-8), stepped on forked streams inside the graph (see
+ *                    (1-8; 0: by the size of the batch, for graphs of
+ *                    one class), stepped on forked streams inside the graph (see
  *                    sddc_graph_create_multi), so that the latency-bound
  *                    solves of one part overlap the transforms of another.
  *                    Results are the same bits as one batch.

@@ -190,6 +190,22 @@ static int alloc_ws(Plan& p, int B) {
   return SDDC_OK;
 }
 
+// Parts of a batch on forked streams in a graph of nplans classes: the plan's
+// tuning, else by the entries B N of a field.  A part's latency-bound solve runs
+// beside another's transforms; smaller parts leave the device idle instead.  us a
+// step with 1, 2, 4 parts (parts of 16 instances or more; N_fm/N_r, B):
+//   float64  128/30 32  51, 55, -      256/30 64  113, 100, 98    512/40 64  324, 303, 296
+//            64/20 64   44, 46, 64     128/30 64   65, 62, 90    256/30 256  264, 237, 231
+//   mixed    64/20 64   37, 41, 49     256/30 64   97, 90, 86-100
+//            512/40 64  247, 230, 228  512/40 256 514, 511, 482
+// The classes of a graph overlap by themselves.
+static int graph_parts(const Plan& p, int B, int nplans) {
+  if (p.tune_sub_batches > 0) return p.tune_sub_batches;
+  const long long entries = (long long)B * p.K * p.nr;
+  if (nplans > 1 || B < 32 || entries < 220000) return 1;
+  return entries < 900000 ? 2 : 4;
+}
+
 static int check_batch(Plan& p, int B) {
   if (B < 0) return fail(SDDC_ERR_INVALID, "negative batch");
   if (B > p.max_batch) return fail(SDDC_ERR_INVALID, "batch exceeds the plan's reserved size");
@@ -248,7 +264,7 @@ int sddc_plan_tuning(const sddc_plan* plan, sddc_tuning* out) {
   *out = sddc_tuning{};
   out->chain_segment = plan->p.seg_m;
   out->solve_instances = plan->p.tune_solve_nbi;
-  out->sub_batches = plan->p.tune_sub_batches;
+  out->sub_batches = graph_parts(plan->p, plan->p.max_batch, 1);
   out->nab2_solve = plan->p.nab2_modal ? 2 : 1;
   out->spectral_instances = plan->p.tune_spectral_nb;
   return SDDC_OK;
@@ -347,7 +363,7 @@ int sddc_plan_create_tuned(const sddc_operators* ops, int precision, int symmetr
     p.nab2_modal = want == 2 ? 1 : 0;
   }
   p.tune_solve_nbi = tuning ? tuning->solve_instances : 0;
-  p.tune_sub_batches = (tuning && tuning->sub_batches > 0) ? tuning->sub_batches : 1;
+  p.tune_sub_batches = tuning ? tuning->sub_batches : 0;
   if ((rc = build_chain(p, ops, max_batch > 0 ? max_batch : 1,
                         tuning ? tuning->chain_segment : 0)))
     return bail(rc);
@@ -801,7 +817,7 @@ int sddc_graph_create_multi(int nplans, sddc_plan* const* plans, const int* B,
   };
   std::vector<Part> parts;
   for (int c = 0; c < nplans; ++c)
-    for (auto [b0, nb] : split_batch(B[c], plans[c]->p.tune_sub_batches))
+    for (auto [b0, nb] : split_batch(B[c], graph_parts(plans[c]->p, B[c], nplans)))
       parts.push_back({sub_plan(plans[c]->p, b0, nb), c, b0, nb});
   const int np = (int)parts.size();
   auto state_of = [&](const Part& pt) {

@@ -135,7 +135,7 @@ struct Plan {
   double* rowval = nullptr;
   double* params = nullptr;    // 2*max_batch: Ra, Ra_s staging
   int tune_solve_nbi = 0;            // instances per solve workgroup, 0 = automatic
-  int tune_sub_batches = 1;          // parts of a batch on forked streams in graphs
+  int tune_sub_batches = 0;          // parts of a batch on forked streams in graphs, 0 = automatic
   int tune_spectral_nb = 0;          // instances per spectral workgroup, 0 = automatic
   size_t ws_bytes = 0;
 };
