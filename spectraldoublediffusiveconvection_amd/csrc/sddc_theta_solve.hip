@@ -38,8 +38,8 @@
 //
 // V, W: 16-row tiles in the fragment order of sddc_frag.h, for 16x16x4 matrix
 // instructions with 16 modes as rows and 16 radial points as columns.  A
-// workgroup takes one tile, or two neighbours, of one chain of one instance;
-// its wavefronts split the tile's columns into kRanges runs.
+// workgroup takes one tile of one chain of one instance; its wavefronts split
+// the tile's columns into kRanges runs.
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -73,38 +73,32 @@ struct ThetaArgs {
 };
 
 constexpr int kRanges = 4;         // runs of a tile's columns
-constexpr int kLoneTiles = 96;     // instances x tiles up to which a workgroup takes one tile
-constexpr int kPair = 2;           // tiles with common runs
 
-// Column groups of the matrices, and run i of the tiles of a pair (the entries
-// left of the pair's diagonal are zero).  All are even, in pairs of groups.
+// Column groups of the matrices, and run i of a tile (the entries left of its
+// diagonal are zero).  All are even, in pairs of groups.
 __host__ __device__ inline int theta_nq(int tiles) { return 2 * tiles; }
 __device__ __forceinline__ int run_begin(int tile, int nq, int i) {
-  const int q0 = 2 * (tile & ~(kPair - 1));
+  const int q0 = 2 * tile;
   return q0 + (nq - q0) / 2 * i / kRanges * 2;
 }
 
-// One run (column groups qa .. qb) of MT tiles times the rows of one chain in
-// memory: row b at in + b*stride, columns 16w + lane % 16 of every w at off[w].
-// An operand of the tiles serves WR column groups, one of the rows MT tiles:
-// the loads of a lone 16x16 tile cost as much as its products.
-template <int WR, int MT>
-__device__ __forceinline__ void run_product(v4d_th (&acc)[MT][WR], const double* tile, int tsize,
+// Column groups qa .. qb of one tile times the rows of one chain in memory: row b
+// at in + b*stride, columns 16w + lane % 16 of every w at off[w].  An operand of
+// the tile serves all WR column groups.
+template <int WR>
+__device__ __forceinline__ void run_product(v4d_th (&acc)[WR], const double* tile,
                                             const double* in, int stride,
                                             const unsigned (&off)[WR], int qa, int qb, int n,
                                             int lane) {
   struct Stage {
-    double2 av[MT][2];
+    double2 av[2];
     double b[2][2][WR];
   } s[2];
   const int kk = 2 * (lane >> 4);
   auto load = [&](Stage& d, int q) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-        d.av[m][i] = *reinterpret_cast<const double2*>(
-            lane_at(tile + (size_t)m * tsize, 1024u * (q + i) + 16u * lane));
+      d.av[i] = *reinterpret_cast<const double2*>(lane_at(tile, 1024u * (q + i) + 16u * lane));
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         // rows past n meet zero columns of the tile: any row of the chain will do
@@ -121,11 +115,9 @@ __device__ __forceinline__ void run_product(v4d_th (&acc)[MT][WR], const double*
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-          for (int w = 0; w < WR; ++w)
-            acc[m][w] = __builtin_amdgcn_mfma_f64_16x16x4f64(h ? d.av[m][i].y : d.av[m][i].x,
-                                                             d.b[i][h][w], acc[m][w], 0, 0, 0);
+        for (int w = 0; w < WR; ++w)
+          acc[w] = __builtin_amdgcn_mfma_f64_16x16x4f64(h ? d.av[i].y : d.av[i].x, d.b[i][h][w],
+                                                        acc[w], 0, 0, 0);
   };
   if (qa >= qb) return;
   load(s[0], qa);
@@ -143,41 +135,39 @@ __device__ __forceinline__ void run_product(v4d_th (&acc)[MT][WR], const double*
 template <int WR>
 constexpr int theta_waves() { return WR < kRanges ? kRanges : WR + 1; }
 
-// MT tiles from `tile` on; put(tile row, column, value) of the sums, from LDS.
-template <int WR, int MT, typename F>
+// Wavefronts per SIMD that the registers of the products must allow.
+template <int NRS>
+constexpr int theta_occupancy() { return NRS <= 40 ? 4 : 2; }
+
+// One tile by kRanges wavefronts, a run each; put(mode, column, value) of the
+// sums, from LDS.
+template <int WR, typename F>
 __device__ __forceinline__ void split_tile(double* xs, const double* mat, const double* in,
                                            int stride, int tile, int nq, int n, int nr, int wave,
                                            int lane, F put) {
-  constexpr int PS = 16 * WR, ROWS = MT * kThetaModes, THREADS = 64 * theta_waves<WR>();
+  constexpr int PS = 16 * WR, THREADS = 64 * theta_waves<WR>();
   if (wave < kRanges) {
     unsigned off[WR];
-    v4d_th acc[MT][WR];
+    v4d_th acc[WR];
 #pragma unroll
     for (int w = 0; w < WR; ++w) {
       const int r = 16 * w + (lane & 15);
       off[w] = 8u * (r < nr ? r : nr - 1);
-#pragma unroll
-      for (int m = 0; m < MT; ++m) acc[m][w] = (v4d_th){0.0, 0.0, 0.0, 0.0};
+      acc[w] = (v4d_th){0.0, 0.0, 0.0, 0.0};
     }
-    // a second tile of a pair starts at its own diagonal
-    int qa = run_begin(tile, nq, wave);
-    qa = qa < 2 * tile ? 2 * tile : qa;
-    run_product<WR, MT>(acc, mat + (size_t)tile * nq * 128, nq * 128, in, stride, off, qa,
-                        run_begin(tile, nq, wave + 1), n, lane);
+    run_product<WR>(acc, mat + (size_t)tile * nq * 128, in, stride, off, run_begin(tile, nq, wave),
+                    run_begin(tile, nq, wave + 1), n, lane);
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int w = 0; w < WR; ++w)
 #pragma unroll
-      for (int w = 0; w < WR; ++w)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          xs[(wave * ROWS + m * kThetaModes + (lane >> 4) + 4 * v) * PS + 16 * w + (lane & 15)] =
-              acc[m][w][v];
+      for (int v = 0; v < 4; ++v)
+        xs[(wave * kThetaModes + (lane >> 4) + 4 * v) * PS + 16 * w + (lane & 15)] = acc[w][v];
   }
   lds_barrier();
-  for (int e = threadIdx.x; e < ROWS * PS; e += THREADS) {
+  for (int e = threadIdx.x; e < kThetaModes * PS; e += THREADS) {
     double sum = 0.0;
 #pragma unroll
-    for (int i = 0; i < kRanges; ++i) sum += xs[i * ROWS * PS + e];
+    for (int i = 0; i < kRanges; ++i) sum += xs[i * kThetaModes * PS + e];
     put(tile * kThetaModes + e / PS, e % PS, sum);
   }
 }
@@ -201,25 +191,25 @@ __device__ __forceinline__ int theta_field(int i, int mask) {
   return f;
 }
 
-// W g: MT tiles of one chain of one instance.
-template <int NRS, int MT>
-__global__ __launch_bounds__(64 * theta_waves<CShape<NRS>::WR>()) void k_theta_forward(
-    ThetaArgs a, int pairs, int items) {
+// W g: one tile of one chain of one instance.
+template <int NRS>
+__global__ __launch_bounds__(64 * theta_waves<CShape<NRS>::WR>(), theta_occupancy<NRS>()) void
+k_theta_forward(ThetaArgs a, int pairs) {
   constexpr int WR = CShape<NRS>::WR;
-  __shared__ double xs[kRanges * MT * kThetaModes * 16 * WR];
-  const int2 item = theta_item(blockIdx.x, items);
+  __shared__ double xs[kRanges * kThetaModes * 16 * WR];
+  const int2 item = theta_item(blockIdx.x, a.tiles);
   if (item.x >= pairs) return;
-  const int type = item.x / a.c.B, b = item.x % a.c.B;
+  const int type = item.x / a.c.B, b = item.x % a.c.B, tile = item.y;
   const int field = theta_field(type, a.c.fields_mask), parity = type & 1, nr = a.c.nr;
   if (parity_is_zero(a.c.symmetric, field, parity)) return;
-  if (field == 0 && (item.y + 1) * MT * kThetaModes <= a.low) return;
+  if (field == 0 && (tile + 1) * kThetaModes <= a.low) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   double* out = a.GH + ((size_t)(2 * field + parity) * a.n * a.c.B + b) * a.rp;
-  split_tile<WR, MT>(xs, a.W[field > 0][parity],
-                     a.c.G + (size_t)b * a.c.gstride + a.c.goff[field] + parity * nr, 2 * nr,
-                     item.y * MT, a.nq, a.n, nr, wave, lane, [&](int m, int r, double v) {
-                       if (m < a.n && r < a.rp) out[(size_t)m * a.c.B * a.rp + r] = r < nr ? v : 0.0;
-                     });
+  split_tile<WR>(xs, a.W[field > 0][parity],
+                 a.c.G + (size_t)b * a.c.gstride + a.c.goff[field] + parity * nr, 2 * nr, tile,
+                 a.nq, a.n, nr, wave, lane, [&](int m, int r, double v) {
+                   if (m < a.n && r < a.rp) out[(size_t)m * a.c.B * a.rp + r] = r < nr ? v : 0.0;
+                 });
 }
 
 // Sets of WR wavefronts in a workgroup of k_theta_blocks.
@@ -243,7 +233,7 @@ k_theta_blocks(ThetaArgs a, int types, int groups) {
   const int type = mg / quads, quad = mg % quads;
   const int field = theta_field(type, a.c.fields_mask), parity = type & 1, nr = a.c.nr;
   if (parity_is_zero(a.c.symmetric, field, parity)) return;
-  if (field == 0 && quad * kEntryModes < a.low / (kPair * kThetaModes) * (kPair * kThetaModes)) return;
+  if (field == 0 && quad * kEntryModes < a.low / kThetaModes * kThetaModes) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int w = wave % S::WR, set = wave / S::WR, t0 = lane >> 4;
   const int b0 = k % groups * 4 * NG, r = 16 * w + (lane & 15), rr = r < nr ? r : nr - 1;
@@ -304,13 +294,13 @@ k_theta_blocks(ThetaArgs a, int types, int groups) {
 }
 
 // The first workgroups: the chain of the low psi rows of one parity and four
-// instances.  The others: MT tiles of V of one chain of one instance, or of the
+// instances.  The others: one tile of V of one chain of one instance, or of the
 // suffix sums of psi (the types behind the fields').
-template <int NRS, int MT, int KD>
-__global__ __launch_bounds__(64 * theta_waves<CShape<NRS>::WR>()) void k_theta_back(
-    ThetaArgs a, int chains, int types, int items) {
+template <int NRS, int KD>
+__global__ __launch_bounds__(64 * theta_waves<CShape<NRS>::WR>(), theta_occupancy<NRS>()) void
+k_theta_back(ThetaArgs a, int chains, int types) {
   using S = CShape<NRS>;
-  constexpr int SUMS = kRanges * MT * kThetaModes * S::WR * 16, LDS = LdsMap<NRS, 1>::SIZE;
+  constexpr int SUMS = kRanges * kThetaModes * S::WR * 16, LDS = LdsMap<NRS, 1>::SIZE;
   __shared__ __align__(16) double xs[LDS > SUMS ? LDS : SUMS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int nr = a.c.nr, t0 = lane >> 4;
@@ -337,31 +327,35 @@ __global__ __launch_bounds__(64 * theta_waves<CShape<NRS>::WR>()) void k_theta_b
       return;
     }
     // the entry state: the lanes of a radial point take every fourth of the
-    // quads' partial sums, kEntryBurst of all four instances in flight
+    // quads' partial sums, kEntryBurst of two instances in flight
     constexpr int kEntryBurst = 6;
     const int quads = (a.n + kEntryModes - 1) / kEntryModes;
     double sf[4] = {0.0, 0.0, 0.0, 0.0}, sb[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int q = a.low / kEntryModes + t0; q < quads; q += 4 * kEntryBurst) {
-      double f[4][kEntryBurst], g[4][kEntryBurst];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int b = 4 * group + i < a.c.B ? 4 * group + i : a.c.B - 1;
-        const double* e = a.EN + ((size_t)b * 2 + parity) * a.tiles * 4 * 2 * S::NRP + rr;
+    for (int i0 = 0; i0 < 4; i0 += 2) {
+      if (4 * group + i0 >= a.c.B) break;
+      for (int q = a.low / kEntryModes + t0; q < quads; q += 4 * kEntryBurst) {
+        double f[2][kEntryBurst], g[2][kEntryBurst];
 #pragma unroll
-        for (int u = 0; u < kEntryBurst; ++u) {
-          const size_t o = (size_t)(q + 4 * u < quads ? q + 4 * u : q) * 2 * S::NRP;
-          f[i][u] = e[o];
-          g[i][u] = e[o + S::NRP];
-        }
-      }
+        for (int i = 0; i < 2; ++i) {
+          const int b = 4 * group + i0 + i < a.c.B ? 4 * group + i0 + i : a.c.B - 1;
+          const double* e = a.EN + ((size_t)b * 2 + parity) * a.tiles * 4 * 2 * S::NRP + rr;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int u = 0; u < kEntryBurst; ++u)
-          if (q + 4 * u < quads) {
-            sf[i] += f[i][u];
-            sb[i] += g[i][u];
+          for (int u = 0; u < kEntryBurst; ++u) {
+            const size_t o = (size_t)(q + 4 * u < quads ? q + 4 * u : q) * 2 * S::NRP;
+            f[i][u] = e[o];
+            g[i][u] = e[o + S::NRP];
           }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int u = 0; u < kEntryBurst; ++u)
+            if (q + 4 * u < quads) {
+              sf[i0 + i] += f[i][u];
+              sb[i0 + i] += g[i][u];
+            }
+      }
     }
     double fe[1] = {0.0}, bfe[1] = {0.0};
 #pragma unroll
@@ -378,38 +372,36 @@ __global__ __launch_bounds__(64 * theta_waves<CShape<NRS>::WR>()) void k_theta_b
     chain_a4<NRS, 1, KD>(a.c, group, wave, row0, n, fe, bfe, xs);
     return;
   }
-  const int2 item = theta_item(blockIdx.x - (chains + 7) / 8 * 8, items);
+  const int2 item = theta_item(blockIdx.x - (chains + 7) / 8 * 8, a.tiles);
   if ((int)blockIdx.x < (chains + 7) / 8 * 8 || item.x >= types * a.c.B) return;
-  const int type = item.x / a.c.B, b = item.x % a.c.B;
+  const int type = item.x / a.c.B, b = item.x % a.c.B, tile = item.y;
   const int nfields = types / 2 - (a.c.P != nullptr ? 1 : 0);
   const bool sums = type / 2 >= nfields;   // P
   const int field = sums ? 0 : theta_field(type, a.c.fields_mask), parity = type & 1;
-  if (field == 0 && (item.y + 1) * MT * kThetaModes <= a.low) return;
+  if (field == 0 && (tile + 1) * kThetaModes <= a.low) return;
   double* x = (sums ? a.c.P + (size_t)b * a.N : a.c.X + (size_t)b * a.c.xstride + a.c.xoff[field]) +
               parity * nr;
   auto put = [&](int m, int r, double v) {
     if (r < nr && m < a.n && (field > 0 || m >= a.low)) x[(size_t)2 * m * nr + r] = v;
   };
   if (parity_is_zero(a.c.symmetric, field, parity)) {
-    for (int e = threadIdx.x; e < MT * kThetaModes * S::WR * 16; e += blockDim.x)
-      put(item.y * MT * kThetaModes + e / (16 * S::WR), e % (16 * S::WR), 0.0);
+    for (int e = threadIdx.x; e < kThetaModes * S::WR * 16; e += blockDim.x)
+      put(tile * kThetaModes + e / (16 * S::WR), e % (16 * S::WR), 0.0);
     return;
   }
-  split_tile<S::WR, MT>(xs, sums ? a.U[parity] : a.V[field > 0][parity],
-                        a.H + (((size_t)b * 3 + field) * 2 + parity) * a.n * nr, nr, item.y * MT,
-                        a.nq, a.n, nr, wave, lane, put);
+  split_tile<S::WR>(xs, sums ? a.U[parity] : a.V[field > 0][parity],
+                    a.H + (((size_t)b * 3 + field) * 2 + parity) * a.n * nr, nr, tile, a.nq, a.n,
+                    nr, wave, lane, put);
 }
 
-template <int NRS, int MT>
+template <int NRS>
 static int launch_theta_t(const ThetaArgs& a, hipStream_t s) {
   using S = CShape<NRS>;
   const int mask = a.c.fields_mask, B = a.c.B;
   const int types = 2 * ((mask & 1) + ((mask >> 1) & 1) + ((mask >> 2) & 1));
   const dim3 threads(64 * theta_waves<S::WR>());
-  const int items = a.tiles / MT;
-  auto grid = [&](int pairs) { return (pairs + 7) / 8 * 8 * items; };
-  hipLaunchKernelGGL((k_theta_forward<NRS, MT>), dim3(grid(types * B)), threads, 0, s, a, types * B,
-                     items);
+  auto grid = [&](int pairs) { return (pairs + 7) / 8 * 8 * a.tiles; };
+  hipLaunchKernelGGL((k_theta_forward<NRS>), dim3(grid(types * B)), threads, 0, s, a, types * B);
   if (int rc = hip_check(hipGetLastError(), "k_theta_forward")) return rc;
   const int quads = (a.n + kEntryModes - 1) / kEntryModes, rows = (types * quads + 7) / 8 * 8;
   auto blocks = [&](auto kernel, int ng) {
@@ -422,20 +414,12 @@ static int launch_theta_t(const ThetaArgs& a, hipStream_t s) {
     return rc;
   const int btypes = types + (a.c.P ? 2 : 0);
   const int chains = (a.low > 0 && (mask & 1)) ? 2 * ((B + 3) / 4) : 0;
-  hipLaunchKernelGGL((k_theta_back<NRS, MT, 2>), dim3((chains + 7) / 8 * 8 + grid(btypes * B)),
-                     threads, 0, s, a, chains, btypes, items);
+  hipLaunchKernelGGL((k_theta_back<NRS, 2>), dim3((chains + 7) / 8 * 8 + grid(btypes * B)),
+                     threads, 0, s, a, chains, btypes);
   return hip_check(hipGetLastError(), "k_theta_back");
 }
 
-template <int NRS>
-static int dispatch_theta(const ThetaArgs& a, hipStream_t s) {
-  return a.c.B * a.tiles <= kLoneTiles ? launch_theta_t<NRS, 1>(a, s) : launch_theta_t<NRS, 2>(a, s);
-}
-
-// Tiles of n = K/2 modes, whole pairs.
-static int theta_tiles(int K) {
-  return (K / 2 + kPair * kThetaModes - 1) / (kPair * kThetaModes) * kPair;
-}
+static int theta_tiles(int K) { return (K / 2 + kThetaModes - 1) / kThetaModes; }
 
 // The workspaces of the solves, for B instances: arrays that are dead by then.
 // W g is at most 24 bytes a mode and radial point (28 in the slabs), the
@@ -468,14 +452,14 @@ int launch_theta_solve(const Plan& p, const ChainArgs& c, bool step, hipStream_t
     a.entry[par] = p.theta + kThetaMats * sz + (size_t)((step ? 0 : 2) + par) * 2 * a.n;
   }
   switch (p.NRS) {
-    case 8: return dispatch_theta<8>(a, s);
-    case 16: return dispatch_theta<16>(a, s);
-    case 24: return dispatch_theta<24>(a, s);
-    case 32: return dispatch_theta<32>(a, s);
-    case 40: return dispatch_theta<40>(a, s);
-    case 48: return dispatch_theta<48>(a, s);
-    case 56: return dispatch_theta<56>(a, s);
-    case 64: return dispatch_theta<64>(a, s);
+    case 8: return launch_theta_t<8>(a, s);
+    case 16: return launch_theta_t<16>(a, s);
+    case 24: return launch_theta_t<24>(a, s);
+    case 32: return launch_theta_t<32>(a, s);
+    case 40: return launch_theta_t<40>(a, s);
+    case 48: return launch_theta_t<48>(a, s);
+    case 56: return launch_theta_t<56>(a, s);
+    case 64: return launch_theta_t<64>(a, s);
     default: return fail(SDDC_ERR_UNSUPPORTED, "unsupported radial size");
   }
 }
