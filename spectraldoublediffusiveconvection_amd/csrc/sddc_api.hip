@@ -191,19 +191,20 @@ static int alloc_ws(Plan& p, int B) {
 }
 
 // Parts of a batch on forked streams in a graph of nplans classes: the plan's
-// tuning, else by the entries B N of a field.  A part's latency-bound solve runs
-// beside another's transforms; smaller parts leave the device idle instead.  us a
-// step with 1, 2, 4 parts (parts of 16 instances or more; N_fm/N_r, B):
-//   float64  128/30 32  51, 55, -      256/30 64  113, 100, 98    512/40 64  324, 303, 296
-//            64/20 64   44, 46, 64     128/30 64   65, 62, 90    256/30 256  264, 237, 231
-//   mixed    64/20 64   37, 41, 49     256/30 64   97, 90, 86-100
-//            512/40 64  247, 230, 228  512/40 256 514, 511, 482
+// tuning, else by the entries B N of a field (float64: twice, for its slower
+// transforms).  A part's latency-bound solve runs beside another's transforms;
+// smaller parts leave the device idle instead, and how far branches overlap
+// varies between processes by 10%, so the lines are where two parts won in all
+// of them.  us a step with 1, 2, 4 parts (N_fm/N_r, B):
+//   float64  128/30 64  65, 62, 90   256/30 64   113, 100, 98   512/40 64  324, 303, 296
+//   mixed    256/30 64  84-97, 90-94, 86-106     512/40 64  220-247, 213-230, 223-228
+//            256/40 256 277, 253, 252            512/40 256 510, 475, 476 (514, 511, 482)
 // The classes of a graph overlap by themselves.
 static int graph_parts(const Plan& p, int B, int nplans) {
   if (p.tune_sub_batches > 0) return p.tune_sub_batches;
-  const long long entries = (long long)B * p.K * p.nr;
-  if (nplans > 1 || B < 32 || entries < 220000) return 1;
-  return entries < 900000 ? 2 : 4;
+  const long long work = (long long)B * p.K * p.nr * (p.precision == SDDC_MIXED ? 1 : 2);
+  if (nplans > 1 || B < 32 || work < 900000) return 1;
+  return work < 4000000 ? 2 : 4;
 }
 
 static int check_batch(Plan& p, int B) {

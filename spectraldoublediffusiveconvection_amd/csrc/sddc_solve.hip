@@ -378,15 +378,17 @@ void pack_frag(const double* A, int nrows, int ncols, int lda, int NRP, int NC,
 
 // The form of a plan's solves: n, the rows of a chain, or less for the
 // eigenbasis of the theta operator (sddc_theta_solve.hip); the value itself
-// stands for nothing else and is reported by sddc_plan_tuning.  Solve of a step
-// on MI355X, chains against eigenbasis:
+// stands for nothing else and is reported by sddc_plan_tuning.  Solve of a step on
+// MI355X, chains against eigenbasis (timed from the host, where three launches
+// cost about 16 us at least and one 8):
 //   N_fm/N_r  64/20   B = 1, 16        12.4, 12.7   17.6, 16.9 us
-//   90/25     B = 1, 16                16.5, 16.7   17.9, 17.0
-//   128/30    B = 1, 16, 64            23.6, 24, 25        17.8, 17.8, 29.5
-//   256/30    B = 1, 16, 64            43.6, 43.9, 45      18.8, 23.9, 52.7
-//   512/40    B = 1, 16, 64            112, 113, 115       25, 53, 157
+//   90/25     B = 1, 16                16.5, 16.7   17.8, 18.4   (a step 37.7 -> 35.5)
+//   128/30    B = 1, 16, 64            23.6, 24, 25        17.7, 18.2, 28.8
+//   256/30    B = 1, 16, 64            43.6, 43.9, 45      18.6, 23.6, 44.3
+//   512/40    B = 1, 16, 64            112, 113, 115       23, 49, 137
 // The chains take as long for 1 instance as for 64, so plans of up to 96
-// instances, which may be called with fewer, keep the eigenbasis.
+// instances, which may be called with fewer, keep the eigenbasis.  Up to 80 modes
+// the chains are as fast, and agree with the sequential recurrence to rounding.
 // SDDC_CHAIN_SEGMENT overrides.  Fixed per plan, so that the bits of a result do
 // not depend on the batch it was computed in.
 static int default_segment(int n, int max_batch) {
@@ -394,7 +396,7 @@ static int default_segment(int n, int max_batch) {
     const int m = std::atoi(env);
     if (m > 0) return m;
   }
-  if (n <= 48 || max_batch > 96) return n;
+  if (n <= 40 || max_batch > 96) return n;
   const double c = max_batch <= 4 ? 1.0 : 2.0;
   int m = (int)std::ceil(c * std::sqrt((double)n));
   m = ((m + 1) / 2) * 2;
