@@ -590,10 +590,7 @@ static int run_steps(Plan& p, int B, const double* Ra, const double* Ra_s, const
 }
 
 // The plan restricted to instances [b0, b0 + nb): operators shared,
-// per-instance workspace offset by b0.  b0 is a multiple of 16, so the solve's
-// segment exit states stay aligned to whole workgroups.  Concurrent parts
-// share only the solve's sink (stores of padded rows, never read for real
-// instances).
+// per-instance workspace offset by b0.  Concurrent parts share nothing they write.
 static Plan sub_plan(const Plan& p, int b0, int nb) {
   Plan v = p;
   const size_t N = (size_t)p.K * p.nr;
@@ -616,9 +613,9 @@ static Plan sub_plan(const Plan& p, int b0, int nb) {
 // Allocation-free step (sddc_step_static): the step's intermediates in one
 // static device array per GPU instead of the plan's workspace.  Every buffer
 // carved from it is written before it is read within a call (suffix sums,
-// linear part, slabs, products, right-hand side, segment exit states; the
-// solve's sink is only written), so nothing in it has to start at zero and
-// a call does not depend on what an earlier call left there.
+// linear part, slabs, products, right-hand side, the solves' use of the dead ones),
+// so nothing in it has to start at zero and a call does not depend on what an
+// earlier call left there.
 // ---------------------------------------------------------------------------
 constexpr size_t kStaticScratchBytes = (size_t)SDDC_STATIC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];

@@ -110,7 +110,7 @@ struct Plan {
   double* vecs = nullptr;      // 8 vectors of length NRP (see VecId)
   // implicit solves: operator data in MFMA fragment order (layout in sddc_frag.h)
   int NRS = 0;                 // nr rounded up to a multiple of 8
-  int seg_m = 0, nseg = 0;     // rows per chain segment, segments per chain
+  int seg_m = 0, nseg = 0;     // chain_segment; 1: chains, more: theta eigenbasis
   double* chain_L[3] = {nullptr, nullptr, nullptr};   // block inverses, K x NRP x NRS
   double* chain_D2 = nullptr;                         // D2 of the A4 solve (one block)
   // the step's solves in the eigenbasis of the theta operator, when set

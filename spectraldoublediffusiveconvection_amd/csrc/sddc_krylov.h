@@ -57,7 +57,7 @@ __device__ __forceinline__ double block_sum(double v, double* tmp) {
 // partial[(b*pstride + i)*gridDim.x + chunk] = V_i[b] . (x[b] - sub[b]) over a
 // chunk, i < nv; V null: (x - sub) . (x - sub).  sub may be null.
 // Grid: (chunks, ceil(nv / kVectors), B).
-template <bool SELF>   // V is null
+template <bool SELF, bool SUB>   // V is null; sub is not
 __global__ __launch_bounds__(kThreads) void k_dots(Basis V, const double* __restrict__ x,
                                                    const double* __restrict__ sub, int n, int nv,
                                                    int pstride, double* __restrict__ partial,
@@ -68,29 +68,26 @@ __global__ __launch_bounds__(kThreads) void k_dots(Basis V, const double* __rest
   if (gate.skips(b)) return;
   const size_t o = (size_t)b * n;
   const int e0 = blockIdx.x * kChunk + threadIdx.x;
-  double xv[E], s[kVectors];
+  // every load before the first use: a launch is one memory latency
+  double xv[E], sv[E], a[SELF ? 1 : kVectors][E], s[kVectors];
 #pragma unroll
   for (int u = 0; u < E; ++u) {
-    const int e = e0 + u * kThreads;
-    xv[u] = e < n ? x[o + e] : 0.0;
+    const int e = e0 + u * kThreads < n ? e0 + u * kThreads : 0;
+    xv[u] = x[o + e];
+    sv[u] = SUB ? sub[o + e] : 0.0;
+    if (!SELF)
+#pragma unroll
+      for (int q = 0; q < kVectors; ++q)
+        a[SELF ? 0 : q][u] = V.at[(i0 + q < nv ? i0 + q : nv - 1) * V.ld + o + e];
   }
-  if (sub)
 #pragma unroll
-    for (int u = 0; u < E; ++u) {
-      const int e = e0 + u * kThreads;
-      xv[u] -= e < n ? sub[o + e] : 0.0;
-    }
+  for (int u = 0; u < E; ++u) xv[u] = e0 + u * kThreads < n ? xv[u] - sv[u] : 0.0;
 #pragma unroll
-  for (int q = 0; q < kVectors; ++q) {
-    const double* v = SELF ? nullptr : V.at + (i0 + q < nv ? i0 + q : nv - 1) * V.ld + o;
+  for (int q = 0; q < (SELF ? 1 : kVectors); ++q) {
     s[q] = 0.0;
 #pragma unroll
-    for (int u = 0; u < E; ++u) {
-      const int e = e0 + u * kThreads;
-      const double a = SELF ? xv[u] : v[e < n ? e : 0];
-      s[q] = e < n ? fma(a, xv[u], s[q]) : s[q];
-    }
-    if (SELF) break;
+    for (int u = 0; u < E; ++u)
+      if (e0 + u * kThreads < n) s[q] = fma(SELF ? xv[u] : a[SELF ? 0 : q][u], xv[u], s[q]);
   }
   // sums over the wavefront: halves exchange vectors first, so that each lane ends
   // with one (vector lane / 8) and 10 exchanges do instead of 48
@@ -206,12 +203,13 @@ __device__ __forceinline__ void scale_update(double* w, int n, double norm) {
 inline int launch_dots(Basis V, const double* x, const double* sub, int n, int nv, int pstride,
                        double* partial, int B, Gate gate, hipStream_t s) {
   const dim3 grid(chunks(n), (nv + kVectors - 1) / kVectors, B);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, V, x, sub, n, nv, pstride, partial, gate);
+  };
   if (V.at)
-    hipLaunchKernelGGL(k_dots<false>, grid, dim3(kThreads), 0, s, V, x, sub, n, nv, pstride,
-                       partial, gate);
+    sub ? run(k_dots<false, true>) : run(k_dots<false, false>);
   else
-    hipLaunchKernelGGL(k_dots<true>, grid, dim3(kThreads), 0, s, V, x, sub, n, nv, pstride, partial,
-                       gate);
+    sub ? run(k_dots<true, true>) : run(k_dots<true, false>);
   return hip_check(hipGetLastError(), "k_dots");
 }
 

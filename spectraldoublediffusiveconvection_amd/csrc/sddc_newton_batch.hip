@@ -10,7 +10,7 @@
 // kernels for all of them, and every vector operation runs over all B with a
 // per-instance gate.  The small least-squares problem of each instance
 // (Hessenberg column, Givens rotations, residual estimate, back substitution)
-// is updated on the device, one thread per instance, so an Arnoldi step needs
+// is updated on the device, so an Arnoldi step needs
 // no copy to the host; the host reads the instances' activity flags (B ints,
 // pinned memory) only every `check_every` Arnoldi steps, at each restart and
 // once per Newton iteration.  An instance that has converged is frozen (its
@@ -175,23 +175,44 @@ __global__ __launch_bounds__(kThreads) void k_givens(
 }
 
 // End of a cycle: y = H(0:jend, 0:jend)^-1 g(0:jend) for instances that ran
-// it; converged when the residual estimate reached the target.
-__global__ void k_backsolve(const double* __restrict__ H, const double* __restrict__ g,
-                            double* __restrict__ y, double* __restrict__ sc,
-                            int* __restrict__ fl, int m, int B) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
+// it; converged when the residual estimate reached the target.  One wavefront per
+// instance, columns from the right: a solved entry is taken off the rows above by
+// the lanes at once, kAhead columns loaded ahead (one thread walking the triangle
+// from memory took 24 us at 25 columns).  LDS: m doubles.
+__global__ __launch_bounds__(64) void k_backsolve(const double* __restrict__ H,
+                                                  const double* __restrict__ g,
+                                                  double* __restrict__ y, double* __restrict__ sc,
+                                                  int* __restrict__ fl, int m) {
+  extern __shared__ double r[];
+  constexpr int kAhead = 8;
+  const int b = blockIdx.x, lane = threadIdx.x;
   int* f = fl + (size_t)b * kNF;
   if (!f[F_CYCLE]) return;
   const double* Hb = H + (size_t)b * (m + 1) * m;
-  const double* gb = g + (size_t)b * (m + 1);
   double* yb = y + (size_t)b * m;
   const int J = f[F_JEND];
-  for (int i = J - 1; i >= 0; --i) {
-    double acc = gb[i];
-    for (int q = i + 1; q < J; ++q) acc -= Hb[(size_t)i * m + q] * yb[q];
-    yb[i] = acc / Hb[(size_t)i * m + i];
+  for (int k = lane; k < J; k += 64) r[k] = g[(size_t)b * (m + 1) + k];
+  for (int i0 = J - 1; i0 >= 0; i0 -= kAhead) {
+    // the lane's first row of the next columns; rows from 64 on are read in place
+    double h[kAhead], hd[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int i = i0 - u < 0 ? 0 : i0 - u;
+      h[u] = Hb[(size_t)(lane < i ? lane : i) * m + i];
+      hd[u] = Hb[(size_t)i * m + i];
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int i = i0 - u;
+      if (i < 0) break;
+      __syncthreads();
+      const double v = r[i] / hd[u];
+      if (lane == 0) yb[i] = v;
+      if (lane < i) r[lane] -= h[u] * v;
+      for (int k = lane + 64; k < i; k += 64) r[k] -= Hb[(size_t)k * m + i] * v;
+    }
   }
+  if (lane != 0) return;
   f[F_RESTARTS] += 1;
   f[F_ACTIVE] = 0;
   if (sc[(size_t)b * kNS + S_RES] <= sc[(size_t)b * kNS + S_TARGET]) f[F_GCONV] = 1;
@@ -400,8 +421,8 @@ int gmres(sddc_newton_batch* k, Ctx& c, const double* Ra, const double* Ras, con
       }
     }
     // y per instance, dv += V y over its own jend columns
-    hipLaunchKernelGGL(k_backsolve, dim3(pgrid(c.B)), dim3(64), 0, s, c.H, c.g, c.y, c.sc, c.fl, m,
-                       c.B);
+    hipLaunchKernelGGL(k_backsolve, dim3(c.B), dim3(64), m * sizeof(double), s, c.H, c.g, c.y, c.sc,
+                       c.fl, m);
     if ((rc = hip_check(hipGetLastError(), "k_backsolve"))) return rc;
     hipLaunchKernelGGL(k_bcombine, dim3(vgrid(c.n), c.B), dim3(kThreads), 0, s, c.dv, c.V, sJ,
                        c.y, m, -1, c.n, 1.0, 1.0, c.fl, (int)F_CYCLE);

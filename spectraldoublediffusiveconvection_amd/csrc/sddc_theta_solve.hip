@@ -33,7 +33,7 @@
 // chain the difference is 2.4e-14, with 64 3e-15; at N_fm = 64, N_r = 20 it is
 // 2e-14 with none; T and S differ by 2e-15 without.  The plan measures it with
 // a seeded right-hand side and takes the fewest rows (in steps of four per
-// parity) that meet its bound.  The low rows run in the second launch beside
+// parity) that meet its bound.  The low rows run in the last launch beside
 // the back products.
 //
 // V, W: 16-row tiles in the fragment order of sddc_frag.h, for 16x16x4 matrix
