@@ -183,7 +183,9 @@ static int alloc_ws(Plan& p, int B) {
   if ((rc = A(&p.slabs, slab_bytes))) return rc;
   if ((rc = A(&p.slabs2, (size_t)B * 7 * N * 8))) return rc;
   if ((rc = A(&p.F, (size_t)B * 4 * N * rs))) return rc;
-  if ((rc = A((void**)&p.rowval, (size_t)B * p.nr * 8))) return rc;
+  // the diagnostics' row values and partial sums: theirs alone, so that they may run
+  // beside a step on another stream
+  if ((rc = A((void**)&p.rowval, (size_t)B * (p.nr + kDiagParts * diag_parts(p)) * 8))) return rc;
   if ((rc = A((void**)&p.params, (size_t)2 * B * 8))) return rc;
   p.ws_bytes = total;
   p.max_batch = B;
@@ -741,7 +743,7 @@ int sddc_diagnostics(sddc_plan* plan, int B, const double* X, double* out, void*
   if ((rc = launch_spectral(p, B, X, p.Pa, nullptr, nullptr, 0, nullptr, p.slabs2, SDDC_FP64,
                             nullptr, nullptr, s)))
     return rc;
-  double* parts = p.L;   // 40 bytes per kDiagEntries entries
+  double* parts = p.rowval + (size_t)B * p.nr;
   if ((rc = launch_ke_rows(p, B, X, p.slabs2, p.rowval, parts, s))) return rc;
   return launch_diag_final(p, B, p.rowval, parts, out, s);
 }
