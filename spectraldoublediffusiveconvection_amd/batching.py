@@ -101,10 +101,27 @@ class Sweep:
         self.classes = OrderedDict()
         for key, insts in groups.items():
             tuning = tuning_table.lookup(key, len(insts), precision) if tuning_table else None
+            if tuning and precision == "mixed" and len(groups) >= 6 and len(insts) <= 10:
+                tuning = self._fewer_launches(key, tuning)
             self.classes[key] = SizeClass(
                 key, [i["X0"] for i in insts], [i["Ra"] for i in insts],
                 [i["Ra_s"] for i in insts], precision=precision, tuning=tuning,
                 symmetric=symmetric)
+
+    @staticmethod
+    def _fewer_launches(key, tuning):
+        """The chains for the small classes of a sweep of many: more classes
+        than hardware queues wait for their launches, of which the theta
+        eigenbasis takes two more a step, though it is faster alone.  us a
+        step, eigenbasis and chains, twelve classes of 64-512 modes: mixed,
+        24, 51, 96 instances 254 and 230, 255 and 235, 261 and 233, and where
+        a process has the graph's branches on queues of their own 195-208 and
+        196-208; float64, 24 and 37 instances 257 and 250, 257 and 262; with
+        512 modes as chains too 245, 254, 271 (mixed)."""
+        n = key[0] // 2
+        if key[0] > 256 or tuning.get("chain_segment", 0) >= n:
+            return tuning
+        return dict(tuning, chain_segment=n, solve_instances=1)
 
     @property
     def n_instances(self):
