@@ -90,11 +90,15 @@ typedef struct sddc_plan sddc_plan;
  *   chain_segment    the form of the solves: at least the rows of a parity
  *                    chain (N_fm/2), one sequential chain; fewer, the
  *                    eigenbasis of the theta operator, in which every mode
- *                    solves by itself (for small and medium batches; equal
- *                    to rounding, about 2e-14 relative at N_fm = 512; an
+ *                    solves by itself (steps of small and medium batches; an
  *                    operator set whose blocks are no polynomials in that
- *                    operator keeps the chains).  The value below N_fm/2
- *                    has no further meaning
+ *                    operator keeps the chains, as sddc_bsub always does).
+ *                    The two differ by no more than either does from the exact
+ *                    solution, for which the blocks' own accuracy counts:
+ *                    relative, 2.5e-14 for a psi right-hand side of all modes,
+ *                    up to 1.5e-13 (N_fm = 128, N_r = 30) or 1.5e-12 (300, 48)
+ *                    for one of a few modes.  The value below N_fm/2 has no
+ *                    further meaning
  *   solve_instances  launch shape of the chains: 1, 2, 4, 5 four instances
  *                    per workgroup; 6, 10 the same with six instead of four
  *                    rows of operator data in flight; 3, 7 four per A4
@@ -173,7 +177,8 @@ int sddc_nlin_fx(sddc_plan* plan, int B, const double* X, double* out, void* str
 int sddc_nlin_dfx(sddc_plan* plan, int B, const double* dv, const double* X,
                   double* out, void* stream);
 
-/* Back substitutions with the plan's pre-inverted blocks.
+/* Back substitutions with the plan's pre-inverted blocks, row by row whatever
+ * the form of the plan's steps (chain_segment).
  *   field 0: A4_BSub_TSTEP_V2 (Matrix_Operators.py:1115-1194), dt = Pr*dt
  *   field 1: NAB2_BSub_TSTEP_V2 (:1033-1086) with Linv_T, dt
  *   field 2: NAB2_BSub_TSTEP_V2 with Linv_S, Tau*dt

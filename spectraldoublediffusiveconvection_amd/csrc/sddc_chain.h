@@ -324,8 +324,7 @@ __device__ __forceinline__ bool parity_is_zero(int symmetric, int field, int par
 }
 
 struct Plan;
-// The solves of c in the theta eigenbasis; step: with the bound of the steps,
-// else with that of the back substitution entry point.
-int launch_theta_solve(const Plan& p, const ChainArgs& c, bool step, hipStream_t s);
+// The solves of c in the theta eigenbasis.
+int launch_theta_solve(const Plan& p, const ChainArgs& c, hipStream_t s);
 
 }  // namespace sddc

@@ -116,7 +116,7 @@ struct Plan {
   // the step's solves in the eigenbasis of the theta operator, when set
   // (sddc_theta_solve.hip): W, V (sine, cosine; even, odd rows), U (sine), entry weights
   double* theta = nullptr;
-  int theta_low[2] = {0, 0};   // psi rows per parity left to the chain: steps, sddc_bsub
+  int theta_low = 0;           // psi rows per parity left to the chain
   // NAB2 solves in the eigenbasis of r^2 - h r^2 Lap (fields 1, 2), when set:
   // per field lam [NRS] (padding 1), V [nr][NRS], V^-1 [NRS][NRS] (padding 0)
   int nab2_modal = 0;

@@ -303,6 +303,8 @@ static int dispatch_chain(const ChainArgs& a, int nrs, int width, hipStream_t s)
   }
 }
 
+// step: a step's solves, in the plan's form; else (sddc_bsub) the chains, which
+// agree with the sequential recurrence to rounding for every right-hand side.
 int launch_solve_ex(const Plan& p, int B, const double* G, long long gstride,
                     const long long goff[3], double* X, long long xstride,
                     const long long xoff[3], double* Pout, int fields_mask, bool step, hipStream_t s) {
@@ -348,7 +350,7 @@ int launch_solve_ex(const Plan& p, int B, const double* G, long long gstride,
     a.fields_mask = fields_mask & 1;
     if (!a.fields_mask) return SDDC_OK;
   }
-  if (p.theta) return launch_theta_solve(p, a, step, s);
+  if (p.theta && step) return launch_theta_solve(p, a, s);
   const int width = p.tune_solve_nbi > 0 ? p.tune_solve_nbi : (B >= 64 ? 3 : 1);
   return dispatch_chain(a, p.NRS, width, s);
 }

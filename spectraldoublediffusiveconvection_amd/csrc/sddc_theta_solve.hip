@@ -25,16 +25,24 @@
 //
 // Accuracy.  The given A4 blocks are inverses to a few digits less than float64
 // (their condition number is up to 1e9 at low modes), and chain and eigenbasis
-// carry that differently: at N_fm = 512, N_r = 40, dt = 5e-3 both are 4.7e-13
-// from the exact solution of the discretised operators and 2.6e-13 from each
-// other.  The difference comes from the lowest modes, so the lowest psi rows
+// carry that differently.  For a right-hand side with all modes, at N_fm = 512,
+// N_r = 40, dt = 5e-3, both are 4.7e-13 from the exact solution of the
+// discretised operators and 2.6e-13 from each other; T and S differ by 2e-15.
+// Most of that comes from the lowest modes, so the lowest psi rows
 // are solved by the chain, entered with the state of the rows above, which is
 // linear in their eigenbasis solution: with 32 of the 512 rows left to the
-// chain the difference is 2.4e-14, with 64 3e-15; at N_fm = 64, N_r = 20 it is
-// 2e-14 with none; T and S differ by 2e-15 without.  The plan measures it with
-// a seeded right-hand side and takes the fewest rows (in steps of four per
-// parity) that meet its bound.  The low rows run in the last launch beside
-// the back products.
+// chain the difference is 2.4e-14; at N_fm = 64, N_r = 20 it is
+// 2e-14 with none.  The plan measures it with a seeded right-hand side of all
+// modes and takes the fewest rows (in steps of four per parity) that meet
+// kStepTol.  That is no bound for every right-hand side: one confined to a few
+// rows above the chain's shows the blocks' own error, 1e-14 to 1.5e-13 from the
+// chain at 128/30 and up to 1.5e-12 at 300/48 (single rows and bands of 4 to 64,
+// dt = 5e-3, 12 low rows).  Against the exact solution the worst such case is the
+// chain's own (chain and this form: 4.7e-13 both at 128/30, 7.7e-12 both at 300/48,
+// 1.1e-12 both at 512/40; single rows between 0.5 and 4.7 times the chain's).  The
+// back substitution entry point (sddc_bsub), whose result is defined by the blocks
+// it is given, therefore takes the chains in every plan.  The low rows run in the
+// last launch beside the back products.
 //
 // V, W: 16-row tiles in the fragment order of sddc_frag.h, for 16x16x4 matrix
 // instructions with 16 modes as rows and 16 radial points as columns.  A
@@ -54,9 +62,10 @@ typedef double v4d_th __attribute__((ext_vector_type(4)));
 constexpr int kThetaModes = 16;    // modes per tile
 constexpr int kEntryModes = 4;     // modes per partial sum of the entry state
 constexpr int kThetaMats = 10;     // W, V: (sine, cosine) x (even, odd rows); U: sine
-// largest relative difference to the chains that the steps and the back
-// substitution entry point allow (see the head of this file)
-constexpr double kStepTol = 2.5e-14, kBsubTol = 5e-15;
+// Largest relative difference to the chains, measured with one right-hand side of
+// all modes (see the head of this file): psi, which takes low rows until it is met,
+// and T and S, which keep the chains where it is not.
+constexpr double kStepTol = 2.5e-14, kHeatTol = 5e-15;
 
 struct ThetaArgs {
   ChainArgs c;
@@ -429,7 +438,7 @@ static bool theta_fits(int K, int nr, int NRP) {
   return nr >= 8 && (size_t)theta_tiles(K) * 4 * 2 * 2 * NRP * 8 <= (size_t)16 * K * nr;
 }
 
-int launch_theta_solve(const Plan& p, const ChainArgs& c, bool step, hipStream_t s) {
+int launch_theta_solve(const Plan& p, const ChainArgs& c, hipStream_t s) {
   ThetaArgs a;
   a.c = c;
   a.GH = static_cast<double*>(p.slabs);
@@ -439,7 +448,7 @@ int launch_theta_solve(const Plan& p, const ChainArgs& c, bool step, hipStream_t
   a.n = p.K / 2;
   a.tiles = theta_tiles(p.K);
   a.nq = theta_nq(a.tiles);
-  a.low = step ? p.theta_low[0] : p.theta_low[1];
+  a.low = p.theta_low;
   a.N = (long long)p.K * p.nr;
   const size_t sz = (size_t)a.tiles * a.nq * 128;
   for (int basis = 0; basis < 2; ++basis)
@@ -449,7 +458,7 @@ int launch_theta_solve(const Plan& p, const ChainArgs& c, bool step, hipStream_t
     }
   for (int par = 0; par < 2; ++par) {
     a.U[par] = p.theta + (size_t)(8 + par) * sz;
-    a.entry[par] = p.theta + kThetaMats * sz + (size_t)((step ? 0 : 2) + par) * 2 * a.n;
+    a.entry[par] = p.theta + kThetaMats * sz + (size_t)par * 2 * a.n;
   }
   switch (p.NRS) {
     case 8: return launch_theta_t<8>(a, s);
@@ -505,15 +514,14 @@ static void theta_basis(int n, int parity, bool cosine, std::vector<double>& V,
 // One seeded right-hand side through the chains and the eigenbasis, on the
 // host.  False when the operator set's blocks are not those of the operators
 // above (the set may hold any matrices; the chains define the result then).
-// Else the numbers of low psi rows per parity that meet the two bounds.  fields:
+// Else the number of low psi rows per parity that meets kStepTol.  fields:
 // those solved with blocks (the modal NAB2 solve leaves psi).
 static bool theta_probe(const sddc_operators* o, int K, int nr, int fields, const double dtf[3],
                         const std::vector<double> (&V)[2][2],
-                        const std::vector<double> (&W)[2][2], int low[2]) {
+                        const std::vector<double> (&W)[2][2], int& low) {
   const int n = K / 2;
   const size_t NN = (size_t)nr * nr;
   const double* inv[3] = {o->Linv_A4, o->Linv_T, o->Linv_S};
-  const double tol[2] = {kStepTol, kBsubTol};
   std::vector<double> g((size_t)n * nr), f(g), h(g), t(g), x(nr);
   unsigned seed = 12345u;
   for (double& e : g) {
@@ -578,7 +586,7 @@ static bool theta_probe(const sddc_operators* o, int K, int nr, int fields, cons
     }
     return f2 > 0.0 ? std::sqrt(d2 / f2) : (d2 == 0.0 ? 0.0 : INFINITY);
   };
-  low[0] = low[1] = 0;
+  low = 0;
   for (int fld = 0; fld < fields; ++fld)
     for (int par = 0; par < 2; ++par) {
       chain(fld, par, n, f);
@@ -589,15 +597,14 @@ static bool theta_probe(const sddc_operators* o, int K, int nr, int fields, cons
       tri(V[fld > 0][par], h, t);
       if (!(diff(t, f) <= 1e-10)) return false;   // NaN counts as a mismatch
       if (fld > 0) {
-        if (diff(t, f) > kBsubTol) return false;
+        if (diff(t, f) > kHeatTol) return false;
         continue;
       }
-      for (int q = 0; q < 2; ++q)
-        for (; low[q] < n; low[q] = std::min(n, low[q] + kEntryModes)) {
-          h = t;
-          chain(0, par, low[q], h);
-          if (diff(h, f) <= tol[q]) break;
-        }
+      for (; low < n; low = std::min(n, low + kEntryModes)) {
+        h = t;
+        chain(0, par, low, h);
+        if (diff(h, f) <= kStepTol) break;
+      }
     }
   return true;
 }
@@ -611,7 +618,7 @@ int build_theta(Plan& p, const sddc_operators* ops) {
     for (int par = 0; par < 2; ++par) theta_basis(n, par, basis == 1, V[basis][par], W[basis][par]);
   const double dtf[3] = {p.Pr * p.dt, p.dt, p.Tau * p.dt};
   if (!theta_probe(ops, p.K, p.nr, p.nab2_modal ? 1 : 3, dtf, V, W, p.theta_low)) return SDDC_OK;   // the chains solve
-  std::vector<double> all(kThetaMats * sz + 8 * (size_t)n, 0.0);
+  std::vector<double> all(kThetaMats * sz + 4 * (size_t)n, 0.0);
   for (int basis = 0; basis < 2; ++basis)
     for (int par = 0; par < 2; ++par) {
       pack_frag(W[basis][par].data(), n, n, n, 16 * tiles, 8 * nq,
@@ -630,15 +637,13 @@ int build_theta(Plan& p, const sddc_operators* ops) {
       }
     }
     pack_frag(U.data(), n, n, n, 16 * tiles, 8 * nq, all.data() + (size_t)(8 + par) * sz);
-    for (int q = 0; q < 2; ++q) {
-      const int top = p.theta_low[q] - 1;
-      if (top < 0) continue;
-      double* e = all.data() + kThetaMats * sz + (size_t)(2 * q + par) * 2 * n;
-      for (int c = top + 1; c < n; ++c) {   // zero for the chain's own rows
-        const double j = par + 2 * c;
-        e[c] = U[(size_t)top * n + c];
-        e[n + c] = -(j + 1) * (j + 2) * e[c];
-      }
+    const int top = p.theta_low - 1;
+    if (top < 0) continue;
+    double* e = all.data() + kThetaMats * sz + (size_t)par * 2 * n;
+    for (int c = top + 1; c < n; ++c) {   // zero for the chain's own rows
+      const double j = par + 2 * c;
+      e[c] = U[(size_t)top * n + c];
+      e[n + c] = -(j + 1) * (j + 2) * e[c];
     }
   }
   SDDC_HIP(hipMalloc(&p.theta, all.size() * sizeof(double)));
