@@ -265,7 +265,7 @@ int sddc_plan_create(const sddc_operators* ops, int precision, int symmetric, in
 int sddc_plan_tuning(const sddc_plan* plan, sddc_tuning* out) {
   if (!plan || !out) return fail(SDDC_ERR_INVALID, "null argument");
   *out = sddc_tuning{};
-  out->chain_segment = plan->p.seg_m;
+  out->chain_segment = plan->p.chain_segment;
   out->solve_instances = plan->p.tune_solve_nbi;
   out->sub_batches = graph_parts(plan->p, plan->p.max_batch, 1);
   out->nab2_solve = plan->p.nab2_modal ? 2 : 1;
@@ -370,7 +370,8 @@ int sddc_plan_create_tuned(const sddc_operators* ops, int precision, int symmetr
   if ((rc = build_chain(p, ops, max_batch > 0 ? max_batch : 1,
                         tuning ? tuning->chain_segment : 0)))
     return bail(rc);
-  if (p.nseg > 1 && (rc = build_theta(p, ops))) return bail(rc);
+  if (p.chain_segment < p.K / 2 && (rc = build_theta(p, ops))) return bail(rc);
+  if (!p.theta) p.chain_segment = p.K / 2;   // the form in use, for sddc_plan_tuning
   if ((rc = build_tables(p.tabM, p.M))) return bail(rc);
   if ((rc = build_tables(p.tabKE, 3 * p.K))) return bail(rc);
   if ((rc = alloc_ws(p, max_batch > 0 ? max_batch : 1))) return bail(rc);

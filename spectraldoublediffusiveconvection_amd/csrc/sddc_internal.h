@@ -110,10 +110,10 @@ struct Plan {
   double* vecs = nullptr;      // 8 vectors of length NRP (see VecId)
   // implicit solves: operator data in MFMA fragment order (layout in sddc_frag.h)
   int NRS = 0;                 // nr rounded up to a multiple of 8
-  int seg_m = 0, nseg = 0;     // chain_segment; 1: chains, more: theta eigenbasis
+  int chain_segment = 0;       // K/2: chains; less: theta eigenbasis
   double* chain_L[3] = {nullptr, nullptr, nullptr};   // block inverses, K x NRP x NRS
   double* chain_D2 = nullptr;                         // D2 of the A4 solve (one block)
-  // the step's solves in the eigenbasis of the theta operator, when set
+  // the step's solves in the eigenbasis of the theta operator; null: chains
   // (sddc_theta_solve.hip): W, V (sine, cosine; even, odd rows), U (sine), entry weights
   double* theta = nullptr;
   int theta_low = 0;           // psi rows per parity left to the chain

@@ -4,7 +4,6 @@
 // Two forms, chosen per plan (chain_segment): the chains of sddc_chain.h over
 // all rows, for batches whose many chains fill the device, and the theta
 // eigenbasis of sddc_theta_solve.hip for smaller ones.
-#include <cmath>
 #include <cstdlib>
 #include <vector>
 
@@ -379,8 +378,8 @@ void pack_frag(const double* A, int nrows, int ncols, int lda, int NRP, int NC,
 }
 
 // The form of a plan's solves: n, the rows of a chain, or less for the
-// eigenbasis of the theta operator (sddc_theta_solve.hip); the value itself
-// stands for nothing else and is reported by sddc_plan_tuning.  Solve of a step on
+// eigenbasis of the theta operator (sddc_theta_solve.hip), where the value itself
+// stands for nothing else.  Solve of a step on
 // MI355X, chains against eigenbasis (timed from the host, where three launches
 // cost about 16 us at least and one 8):
 //   N_fm/N_r  64/20   B = 1, 16        12.4, 12.7   17.6, 16.9 us
@@ -398,11 +397,7 @@ static int default_segment(int n, int max_batch) {
     const int m = std::atoi(env);
     if (m > 0) return m;
   }
-  if (n <= 40 || max_batch > 96) return n;
-  const double c = max_batch <= 4 ? 1.0 : 2.0;
-  int m = (int)std::ceil(c * std::sqrt((double)n));
-  m = ((m + 1) / 2) * 2;
-  return m < 8 ? 8 : m;
+  return n <= 40 || max_batch > 96 ? n : 8;
 }
 
 template <typename T>
@@ -416,10 +411,8 @@ int build_chain(Plan& p, const sddc_operators* ops, int max_batch, int segment) 
   const int K = p.K, nr = p.nr, NRS = p.NRS, NRP = p.NRP;
   const size_t BLK = (size_t)NRP * NRS, NN = (size_t)nr * nr;
   const int n = K / 2;   // rows per chain (K is even)
-  int m = segment > 0 ? segment : default_segment(n, max_batch);
-  if (m > n) m = n;
-  p.seg_m = m;
-  p.nseg = (n + m - 1) / m;
+  p.chain_segment = segment > 0 ? segment : default_segment(n, max_batch);
+  if (p.chain_segment > n) p.chain_segment = n;
   const double* inv[3] = {ops->Linv_A4, ops->Linv_T, ops->Linv_S};
   const int nfb = p.nab2_modal ? 1 : 3;   // fields solved with per-mode blocks
   std::vector<double> buf((size_t)(K + kFeedPad) * BLK, 0.0);
