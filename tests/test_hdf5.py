@@ -168,3 +168,28 @@ def test_dropin_checkpoints_have_the_reference_groups(tmp_path):
         r = subprocess.run([PY_H5, "-c", DUMP, fc], capture_output=True, text=True, timeout=120)
         assert r.returncode == 0, r.stderr
         assert json.loads(r.stdout)["Bifurcation/KE"]["value"] == [3.0, 4.0]
+
+
+@pytest.mark.parametrize("path", ["missing", "not a library"])
+def test_files_without_the_library(tmp_path, monkeypatch, path):
+    """Checkpoints are written and read where libsddc.so is not built or does not
+    load, byte for byte as with it."""
+    with_lib, without = str(tmp_path / "a.h5"), str(tmp_path / "b.h5")
+    _hdf5.write(with_lib, _tree())
+    lib = tmp_path / "libsddc.so"
+    if path != "missing":
+        lib.write_bytes(b"no library")
+    monkeypatch.setattr(_hdf5._lib, "_lib", None)
+    monkeypatch.setattr(_hdf5._lib, "LIB_PATH", str(lib))
+    with pytest.raises((ImportError, OSError)):
+        _hdf5._lib.lib()
+    _hdf5.write(without, _tree())
+    assert open(with_lib, "rb").read() == open(without, "rb").read()
+    assert _hdf5.read(without)["Parameters"]["N_fm"] == 512
+
+
+@pytest.mark.parametrize("n", [0, 1, 11, 12, 13, 23, 24, 25, 300])
+def test_lookup3_forms_agree(n):
+    k = bytes(np.random.default_rng(n).integers(0, 256, n, dtype=np.uint8))
+    for init in (0, 1, 0xFFFFFFFF):
+        assert _hdf5._lookup3(k, init) == _hdf5.lookup3(k, init)
