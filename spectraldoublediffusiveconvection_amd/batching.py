@@ -101,8 +101,9 @@ class Sweep:
         self.classes = OrderedDict()
         for key, insts in groups.items():
             tuning = tuning_table.lookup(key, len(insts), precision) if tuning_table else None
-            if tuning and precision == "mixed" and len(groups) >= 6 and len(insts) <= 10:
-                tuning = self._fewer_launches(key, tuning)
+            if ((tuning is None or precision == "mixed") and len(groups) >= 6
+                    and len(insts) <= 10):
+                tuning = self._fewer_launches(key, tuning or {})
             self.classes[key] = SizeClass(
                 key, [i["X0"] for i in insts], [i["Ra"] for i in insts],
                 [i["Ra_s"] for i in insts], precision=precision, tuning=tuning,
@@ -110,14 +111,23 @@ class Sweep:
 
     @staticmethod
     def _fewer_launches(key, tuning):
-        """The chains for the small classes of a sweep of many: more classes
-        than hardware queues wait for their launches, of which the theta
-        eigenbasis takes two more a step, though it is faster alone.  us a
-        step, eigenbasis and chains, twelve classes of 64-512 modes: mixed,
-        24, 51, 96 instances 254 and 230, 255 and 235, 261 and 233, and where
-        a process has the graph's branches on queues of their own 195-208 and
-        196-208; float64, 24 and 37 instances 257 and 250, 257 and 262; with
-        512 modes as chains too 245, 254, 271 (mixed)."""
+        """The chains for the small classes of a sweep of many: classes on the
+        same hardware queue (four, by default) wait for each other's launches, of
+        which the theta eigenbasis takes two more a step, though it is faster
+        alone.  For entries of the mixed table and for classes without an entry
+        (an entry of another table stands in float64).  us a step, eigenbasis and
+        chains up to 256 modes, four processes, which differ in how the graph's
+        branches share queues (classes of 64-512 modes x instances each):
+          4 x 2   mixed 69-76, 73       float64 61-72, 75
+          5 x 2   mixed 83-89, 80-89    float64 83-90, 83-86
+          6 x 1   mixed 90-106, 84-88   float64 85-105, 86-89
+          8 x 8   mixed 148-158, 135-143  float64 156-160, 147-152
+          12 x 1  mixed 174-224, 184-195  float64 214-228, 188-200
+          12 x 4  mixed 210-233, 202-210  float64 220-231, 209-212
+          12 x 12 mixed 236-240, 244-248  float64 279-283, 278-286
+        (six classes of 64 and 256 modes alone, two each: mixed 88-104, 104-106.)
+        So a class's form, and with it the last bits of its results, depends on how
+        many classes and instances its sweep has."""
         n = key[0] // 2
         if key[0] > 256 or tuning.get("chain_segment", 0) >= n:
             return tuning

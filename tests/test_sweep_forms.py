@@ -50,3 +50,39 @@ def test_sweep_of_many_small_classes(classes, each, precision, chains):
             x = O.step(x, o, inst["Ra"], inst["Ra_s"])
         e = np.linalg.norm(got[i] - x) / np.linalg.norm(x)
         assert e < (2e-5 if precision == "mixed" else 1e-12), (i, e)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("classes,each,precision,chains", [(6, 1, "fp64", True), (5, 1, "fp64", False),
+                                                           (6, 11, "fp64", False),
+                                                           (6, 1, "mixed", True)])
+def test_sweep_without_table_entries(classes, each, precision, chains):
+    """The same lines for classes that the table has no entry for: a float64 sweep
+    of many small classes waits for its launches as a mixed one does."""
+    sizes = [(258 if i == 0 else 98 + 12 * i, 12 + i) for i in range(classes)]
+    rng = np.random.default_rng(classes + each)
+    insts = []
+    for K, Nr in sizes * each:
+        x = rng.standard_normal(3 * K * (Nr - 1))
+        insts.append(dict(N_fm=K, N_r=Nr, d=0.35, dt=5e-3, Pr=1.0, Tau=1 / 15.0,
+                          Ra=float(rng.uniform(2500, 3000)), Ra_s=500.0,
+                          X0=1e-3 * x / np.linalg.norm(x)))
+
+    class Table:
+        def lookup(self, key, B, precision):
+            return None
+    for table in (None, Table()):
+        sw = batching.Sweep(insts, precision=precision, tuning_table=table)
+        for (K, *_), c in sw.classes.items():
+            assert (c.plan.tuning()["chain_segment"] == K // 2) == (chains and K <= 256), K
+        g = sw.graph(nsteps=2)
+        g.launch()
+        got = sw.states()
+        g.close()
+        for i in range(classes):
+            o = O.build_operators(*batching.class_key(insts[i]))
+            x = insts[i]["X0"]
+            for _ in range(2):
+                x = O.step(x, o, insts[i]["Ra"], insts[i]["Ra_s"])
+            e = np.linalg.norm(got[i] - x) / np.linalg.norm(x)
+            assert e < (2e-5 if precision == "mixed" else 1e-12), (i, e)
