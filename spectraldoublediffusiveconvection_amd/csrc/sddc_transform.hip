@@ -276,12 +276,22 @@ int launch_transform(const TableSet& t, int kind, int rows, int len_in, int n_ou
     auto run = [&](auto launch) { return launch(t, kind, rows, len_in, n_out, in, out, s); };
     // Few rows leave SIMDs idle: four wavefronts share a transform.  Many rows: one,
     // without workgroup barriers, while its registers leave room for others (8
-    // columns); longer ones keep k_transform.  One transform, us, before and now:
+    // columns); longer ones keep k_transform.  One transform, us, k_transform and now:
     //   length   24   96  192  384  450  768  810
     //   1 row   4.7  5.2  5.5  6.4  6.6  7.4  9.2   4.6  4.4  4.2  4.4  5.4  4.7  7.3
     //   2496    6.5  7.3  7.9 11.1 12.2 16.1 19.7   4.5  5.1  5.1  8.6 11.9 13.5 19.7
     //   10000    18   22   24   35   40   52   62   5.7  8.6  9.3   18   28   32   62
-    const bool few = rows <= 2048;
+    // The line: two workgroups of four wavefronts on each CU take 1024 rows.  At
+    // 1024 and 1400 rows, four against one wavefront 300: 6.6, 6.4 and 7.9, 6.5,
+    // 450: 7.3, 7.9 and 9.1, 8.3; four against k_transform 600: 9.4, 9.6 and 11.4,
+    // 10.7, 1080: 14.0, 14.0 and 20, 16.  With 13 to 16 columns four stay level with
+    // k_transform to 2048 rows (960: 11.1, 11.8 and at 2048 16.1, 16.1), and above 16
+    // where k_transform's LDS no longer holds the rows at once (1280: 1400 rows 20,
+    // 17, 1800 rows 24, 26.5; 1728: 26.5, 33 and 31, 37).  768 alone: at 2048 rows
+    // 11.1, 9.1, at 2500 12.6, 13.1, at 4096 17.3, 14.6, everywhere below
+    // k_transform (12.9, 15, 23.5).
+    const int at_once = 512 * (int)(160 * 1024 / (2 * (size_t)t.L * sizeof(double2) + 256));
+    const bool few = rows <= 1024 || (rows <= 2048 && (nc > 16 ? rows > at_once : nc > 12));
     if (t.L == 192) return run(launch_transform_nc<3, 1, 192>);
     if (t.L == 384)
       return few ? run(launch_transform_nc<2, 4, 384>) : run(launch_transform_nc<6, 1, 384>);

@@ -37,3 +37,20 @@ def test_transforms_at_length(L, rows):
         ref = [O.idct(a[b], L), O.idst(a[b], L), O.dct(x[b])[:K], O.dst(x[b])[:K]]
         for g, r in zip(got, ref):
             assert np.linalg.norm(g[b] - r) < 1e-14 * np.linalg.norm(r), b
+
+
+# on both sides of the row counts at which the kernel changes: 4-8, 9-12, 13-16 and
+# more columns, with three, four and two workgroups of k_transform on a CU
+@pytest.mark.parametrize("L", [300, 384, 600, 810, 1080, 1280, 1728])
+@pytest.mark.parametrize("rows", [1024, 1025, 1535, 1537, 2048])
+def test_transforms_around_the_row_lines(L, rows):
+    """1e-14 of each row's norm, as above, for the first and last rows."""
+    K = 2 * L // 3
+    rng = np.random.default_rng(L + rows)
+    a, x = rng.standard_normal((rows, K)), rng.standard_normal((rows, L))
+    got = [run(_lib.SDDC_IDCT, a, L), run(_lib.SDDC_IDST, a, L), run(_lib.SDDC_DCT, x, K),
+           run(_lib.SDDC_DST, x, K)]
+    for b in (0, 1, rows - 2, rows - 1):
+        ref = [O.idct(a[b], L), O.idst(a[b], L), O.dct(x[b])[:K], O.dst(x[b])[:K]]
+        for g, r in zip(got, ref):
+            assert np.linalg.norm(g[b] - r) < 1e-14 * np.linalg.norm(r), b
