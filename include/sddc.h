@@ -333,8 +333,10 @@ int sddc_arclength_step(sddc_krylov* k, const double* Ra_s, double* Y, double* Y
 /* Launch one stage of the step on the plan's workspace (for timing and
  * profiling; no counterpart in the reference).  stage: 0 suffix sums,
  * 1 spectral stage, 2 nonlinear products, 3 right-hand side, 4 solves.
- * X is the state read by stages 0-1; stage 4 writes into plan scratch.  A
- * full sddc_step on the same batch must have run first. */
+ * X is the state read by stages 0-1; stage 4 writes into plan scratch, and in
+ * plans that solve in the eigenbasis (chain_segment below N_fm/2) also over what
+ * stages 2 and 3 read: behind a stage 4 run stage 1 again before them if their
+ * values matter.  A full sddc_step on the same batch must have run first. */
 int sddc_run_stage(sddc_plan* plan, int B, int stage, const double* X, const double* Ra,
                    const double* Ra_s, void* stream);
 

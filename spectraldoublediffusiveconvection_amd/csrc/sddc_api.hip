@@ -201,6 +201,11 @@ static int alloc_ws(Plan& p, int B) {
 //   float64  128/30 64  65, 62, 90   256/30 64   113, 100, 98   512/40 64  324, 303, 296
 //   mixed    256/30 64  84-97, 90-94, 86-106     512/40 64  220-247, 213-230, 223-228
 //            256/40 256 277, 253, 252            512/40 256 510, 475, 476 (514, 511, 482)
+// Around the lines (work in thousands), 1, 2, 4 parts, where two processes agreed to 2%:
+//   712  float64 128/30 96  78, 77, 81     256/30 48  88, 86, 88   mixed 256/30 96 116, 110, 113
+//   950  mixed 256/30 128 117, 120, 121    512/40 48  174, 171, 170    300/48 64 212, 196, 190
+//   2555, 3194, 3993  mixed 512/40 128 320, 308, 294   160 357, 359, 346   200 434, 428, 403
+//   3833, 5111  float64 512/40 96 441, 421, 416   128 459, 454, 403
 // The classes of a graph overlap by themselves.
 static int graph_parts(const Plan& p, int B, int nplans) {
   if (p.tune_sub_batches > 0) return p.tune_sub_batches;

@@ -387,8 +387,12 @@ void pack_frag(const double* A, int nrows, int ncols, int lda, int NRP, int NC,
 //   128/30    B = 1, 16, 64            23.6, 24, 25        17.7, 18.2, 28.8
 //   256/30    B = 1, 16, 64            43.6, 43.9, 45      18.6, 23.6, 44.3
 //   512/40    B = 1, 16, 64            112, 113, 115       23, 49, 137
-// The chains take as long for 1 instance as for 64, so plans of up to 96
-// instances, which may be called with fewer, keep the eigenbasis.  Up to 80 modes
+// The chains take as long for 1 instance as for 64, and a plan may be called with
+// fewer instances than it has room for, so the line of 96 trades one for the other:
+// full batches of 65 to 96 would be faster with the chains (a float64 step, chains
+// and eigenbasis, 65 and 96 instances: 128/30 64, 68 and 72, 80 us, 300/48 267, 284
+// and 362, 402, 512/40 298, 320 and 386, 459), single instances slower (512/40 solve
+// 112 and 23).  Up to 80 modes
 // the chains are as fast, and agree with the sequential recurrence to rounding.
 // SDDC_CHAIN_SEGMENT overrides.  Fixed per plan, so that the bits of a result do
 // not depend on the batch it was computed in.

@@ -123,7 +123,9 @@ def _Time_Step(X, Ra, Ra_s, Tau, Pr, d, N_fm, N_r, symmetric, save_filename='Tim
                start_time=0, Total_time=1, dt=1e-04, linear=False, Verbose=False):
     """Integrate Total_time/dt steps of Step_Python with the loop's symmetry
     mask, diagnostics every step and a checkpoint every tenth of the run
-    (Main.py:228-329).  Returns the last state."""
+    (Main.py:228-329).  Returns the last state.  The average step time that it
+    prints at the end is that of the steps on the device's stream (events around
+    each step), where the reference prints the host's time of a step."""
     plan = _reg.step_plan(N_fm, N_r, d, dt, Pr, Tau, symmetric)
     N_iters = int(Total_time / dt)
     N_save = max(int(N_iters / 10), 1)
